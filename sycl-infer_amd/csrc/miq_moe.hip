@@ -34,10 +34,101 @@ __device__ __forceinline__ float block_max256(float v, float *red) {
     return v;
 }
 
-__global__ __launch_bounds__(256) void route_kernel(const float *__restrict__ x, int x_stride,
-                                                    const float *__restrict__ gate_inp, int n_embd, int n_expert,
-                                                    int top_k, float *__restrict__ logits, int32_t *__restrict__ ids,
-                                                    float *__restrict__ wts) {
+// Router logits: logits[t][e] = (float) sum_k gate_inp[e][k] * x[t][k], the
+// reference's F32 router dot (moe.cpp:84-88), a serial double-precision sum in
+// k order.  Each product of two floats is exact in double, so every partial
+// sum rounds as the reference's does and the logit is its value bit for bit.
+// A workgroup owns one token and 64 experts.  The chain of dependent adds is
+// the bound, so nothing else is on it: waves 1..4 load 16 rows each, 256-byte
+// runs of a row per 16 lanes, three 64-value chunks ahead, and leave the
+// products in LDS ([value][expert], two chunks); wave 0, lane = expert, only
+// reads and adds.  Values past the row's end are products of 0 (a sum that
+// starts at +0 does not change by adding them).  16 tokens x 256 experts x
+// 2048 values: 27 us, about 30 clocks per dependent add; one thread per expert
+// with its loads on the chain took 280 us.
+constexpr int kRlC = 64;  // values per chunk
+template <bool VEC>       // 16-byte loads (n_embd % 4 == 0, gate_inp and x 16-byte aligned)
+__global__ __launch_bounds__(320) void route_logits_kernel(const float *__restrict__ x, int x_stride,
+                                                           const float *__restrict__ gate_inp, int n_embd, int n_expert,
+                                                           float *__restrict__ logits) {
+    __shared__ double prod[2][kRlC][65];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int e0 = blockIdx.x * 64, t = blockIdx.y;
+    const int nc = (n_embd + kRlC - 1) / kRlC;
+    const int kl = 4 * (lane & 15), rl = 16 * (wave - 1) + (lane >> 4);  // this lane's values and first row
+    const float *xr = x + (size_t)t * x_stride;
+    struct Piece {
+        float4 w[4], x;
+    } r[3];
+    auto load4 = [&](const float *p, int k) {
+        const int m = n_embd - 1;
+        if constexpr (VEC) return *reinterpret_cast<const float4 *>(p + (k < m ? k : m - 3));
+        else return make_float4(p[k < m ? k : m], p[k + 1 < m ? k + 1 : m], p[k + 2 < m ? k + 2 : m], p[k + 3 < m ? k + 3 : m]);
+    };
+    auto load = [&](Piece &q, int c) {
+        const int k = (c < nc ? c : nc - 1) * kRlC + kl;
+        q.x = load4(xr, k);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int e = e0 + rl + 4 * i;
+            q.w[i] = load4(gate_inp + (size_t)(e < n_expert ? e : n_expert - 1) * n_embd, k);
+        }
+    };
+    auto produce = [&](const Piece &q, int c) {
+        const float xv[4] = {q.x.x, q.x.y, q.x.z, q.x.w};
+        bool in[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) in[v] = c * kRlC + kl + v < n_embd;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float wv[4] = {q.w[i].x, q.w[i].y, q.w[i].z, q.w[i].w};
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                prod[c & 1][kl + v][rl + 4 * i] = (double)(in[v] ? wv[v] : 0.0f) * (double)(in[v] ? xv[v] : 0.0f);
+        }
+    };
+    // one barrier per chunk on both sides: chunk c is in LDS, chunk c-1 is added
+    if (wave) {
+#pragma unroll
+        for (int j = 0; j < 3; j++) load(r[j], j);
+        produce(r[0], 0);
+        load(r[0], 3);
+        for (int c0 = 0; c0 < nc; c0 += 3) {
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                const int c = c0 + j;
+                if (c >= nc) break;
+                __syncthreads();
+                produce(r[(j + 1) % 3], c + 1);  // past the last chunk: zeros into the slot that is done
+                load(r[(j + 1) % 3], c + 4);
+            }
+        }
+        return;
+    }
+    double a = 0.0;
+    for (int c = 0; c < nc; c++) {
+        __syncthreads();
+        // sixteen reads ahead of the sixteen adds they feed
+        const double *p = &prod[c & 1][0][lane];
+        double v[2][16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) v[0][i] = p[i * 65];
+#pragma unroll
+        for (int b = 0; b < kRlC / 16; b++) {
+            if (b + 1 < kRlC / 16)
+#pragma unroll
+                for (int i = 0; i < 16; i++) v[(b + 1) & 1][i] = p[(16 * (b + 1) + i) * 65];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 16; i++) a += v[b & 1][i];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    if (e0 + lane < n_expert) logits[(size_t)t * n_expert + e0 + lane] = (float)a;
+}
+
+__global__ __launch_bounds__(256) void route_kernel(int n_expert, int top_k, float *__restrict__ logits,
+                                                    int32_t *__restrict__ ids, float *__restrict__ wts) {
     extern __shared__ __align__(16) float sp[];  // [n_expert rounded to 4] probabilities
     __shared__ float red[4];
     __shared__ float s_inv, s_den;
@@ -45,20 +136,6 @@ __global__ __launch_bounds__(256) void route_kernel(const float *__restrict__ x,
     const int t = blockIdx.x;
     const int ne4 = (n_expert + 3) & ~3;
     float *lg = logits + (size_t)t * n_expert;
-    if (gate_inp) {
-        // one thread per expert: the reference's F32 router dot (moe.cpp:84-88),
-        // a serial double-precision sum in k order.  Each product of two floats
-        // is exact in double, so every partial sum rounds as the reference's
-        // does and the logit is its value bit for bit.
-        const float *xr = x + (size_t)t * x_stride;
-        for (int e = threadIdx.x; e < n_expert; e += blockDim.x) {
-            const float *w = gate_inp + (size_t)e * n_embd;
-            double a = 0.0;
-            for (int k = 0; k < n_embd; k++) a += (double)w[k] * (double)xr[k];
-            lg[e] = (float)a;
-        }
-        __syncthreads();
-    }
     float mx = -3.402823466e38f;
     for (int e = threadIdx.x; e < ne4; e += blockDim.x) {
         const float v = e < n_expert ? lg[e] : -3.402823466e38f;
@@ -1165,7 +1242,18 @@ int miq_moe_route(hipStream_t stream, const float *x, int x_stride, const float 
     }
     const int V = (n_expert + 63) / 64;
     const dim3 wgrid((n_tok + 3) / 4), wblock(256);
-    if (!gate_inp && V <= 8) {  // given logits, up to 512 experts: one wave per token
+    if (gate_inp) {
+        for (int t0 = 0; t0 < n_tok; t0 += 65535) {  // tokens per launch: the grid's y limit
+            const dim3 grid(V, n_tok - t0 < 65535 ? n_tok - t0 : 65535);
+            const float *xt = x + (size_t)t0 * x_stride;
+            float *lt = logits + (size_t)t0 * n_expert;
+            if (n_embd % 4 == 0 && x_stride % 4 == 0 && (uintptr_t)gate_inp % 16 == 0 && (uintptr_t)xt % 16 == 0)
+                hipLaunchKernelGGL(miq::route_logits_kernel<true>, grid, dim3(320), 0, stream, xt, x_stride, gate_inp, n_embd, n_expert, lt);
+            else
+                hipLaunchKernelGGL(miq::route_logits_kernel<false>, grid, dim3(320), 0, stream, xt, x_stride, gate_inp, n_embd, n_expert, lt);
+        }
+    }
+    if (V <= 8) {  // up to 512 experts: one wave per token
         const int vv = V == 1 ? 1 : V == 2 ? 2 : V <= 4 ? 4 : 8;
         const size_t rl = miq::route_lds_bytes(vv, 4);
         if (vv == 1) hipLaunchKernelGGL(miq::route_wave_kernel<1>, wgrid, wblock, rl, stream, n_tok, n_expert, top_k, logits, ids, wts);
@@ -1173,8 +1261,7 @@ int miq_moe_route(hipStream_t stream, const float *x, int x_stride, const float 
         else if (vv == 4) hipLaunchKernelGGL(miq::route_wave_kernel<4>, wgrid, wblock, rl, stream, n_tok, n_expert, top_k, logits, ids, wts);
         else hipLaunchKernelGGL(miq::route_wave_kernel<8>, wgrid, wblock, rl, stream, n_tok, n_expert, top_k, logits, ids, wts);
     } else {
-        hipLaunchKernelGGL(miq::route_kernel, dim3(n_tok), dim3(256), lds, stream, x, x_stride, gate_inp, n_embd,
-                           n_expert, top_k, logits, ids, wts);
+        hipLaunchKernelGGL(miq::route_kernel, dim3(n_tok), dim3(256), lds, stream, n_expert, top_k, logits, ids, wts);
     }
     return miq::check_launch("miq_moe_route");
 }

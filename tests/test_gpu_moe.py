@@ -59,6 +59,27 @@ def test_route_gate_inp_near_ties(miq, oracle, dev):
     assert bits_equal(lg.cpu().numpy(), eprobs)
 
 
+@pytest.mark.parametrize("n_tok,n_expert,n_embd,top_k", [
+    (1, 8, 1, 2), (3, 64, 63, 4), (2, 65, 64, 8), (5, 130, 65, 8), (2, 600, 196, 10), (4, 63, 2052, 6), (2, 256, 4098, 8)])
+@pytest.mark.parametrize("pad", [0, 1, 4])
+def test_route_gate_inp_sizes(miq, oracle, dev, n_tok, n_expert, n_embd, top_k, pad):
+    """Router logits around the kernel's 64-expert and 64-value tiles, with row strides
+    and lengths that allow 16-byte loads and ones that do not: ids, weights and
+    probabilities equal the oracle's serial double sum bit for bit."""
+    import torch
+    rng = np.random.default_rng(n_expert * 1000 + n_embd)
+    gi = rng.standard_normal((n_expert, n_embd)).astype(np.float32)
+    xp = rng.standard_normal((n_tok, n_embd + pad)).astype(np.float32)
+    lg = torch.zeros((n_tok, n_expert), dtype=torch.float32, device=dev)
+    ids, wts = miq.moe_route(lg, top_k, x=to_dev(xp, dev)[:, :n_embd], gate_inp=to_dev(gi, dev))
+    torch.cuda.synchronize()
+    eids, ewts, eprobs = oracle.moe_route(np.zeros((n_tok, n_expert), np.float32), top_k,
+                                          x=np.ascontiguousarray(xp[:, :n_embd]), gate_inp=gi)
+    assert np.array_equal(ids.cpu().numpy(), eids)
+    assert bits_equal(wts.cpu().numpy(), ewts)
+    assert bits_equal(lg.cpu().numpy(), eprobs)
+
+
 def test_route_config5(miq, oracle, dev):
     """16 tokens, 256 experts, top-8 from N(0,1) logits (config 5)."""
     import torch
