@@ -110,6 +110,8 @@ struct StaticMode {
 };
 }  // namespace
 
+bool static_scratch_mode() { return g_static_mode; }
+
 static int static_scratch_get(hipStream_t stream, size_t part_bytes, size_t n_cnt, float **part, uint32_t **cnt) {
     if (part_bytes > kStaticPartBytes || n_cnt > kStaticCnt) {
         set_error("miq_i8_gemm_noalloc: the shape needs %zu bytes of partials and %zu counters, beyond the static "

@@ -14,6 +14,8 @@ int scratch_get(hipStream_t stream, size_t part_bytes, size_t n_cnt, float **par
 // allocation is zero-filled (arrival counters that their users return to zero).
 enum { kWsPrefill = 0, kWsPrefillCnt = 1, kWsW4Part = 2, kWsSlots = 4 };
 int workspace_get(hipStream_t stream, int slot, size_t bytes, void **ptr, bool zero = false);
+// Inside miq_i8_gemm_noalloc: scratch comes from the static array, a workspace is refused.
+bool static_scratch_mode();
 // Tuning switches (A/B forms of the kernels).  Each starts from the
 // environment variable MIQ_<name>, read once per process, else its default;
 // miq_set_switch() changes it at run time.
@@ -55,6 +57,10 @@ int launch_mfma32(hipStream_t stream, const miq_seg *s, int TB, int32_t *dots = 
 bool pf16_serves(const miq_seg *s);
 bool pf16_prefers(const miq_seg *s, int TB);
 int launch_pf16(hipStream_t stream, const miq_seg *s, int TB);
+bool pfr_serves(const miq_seg *s);
+bool pfr_prefers(const miq_seg *s, int TB);
+int launch_pfr(hipStream_t stream, const miq_seg *segs, int n_segs, int TB);
+int launch_pfr_dots(hipStream_t stream, const miq_seg *s, int TB, int32_t *out);
 int launch_pf16_dots(hipStream_t stream, const miq_seg *s, int TB, int32_t *out);
 
 

@@ -411,6 +411,52 @@ def test_gemm_cu_form_default_many_tiles(miq, oracle, dev):
     assert_elem(out, exp, elem_bound(oracle, Q6_K, wq, K, act, 1.0), residual=None)
 
 
+@pytest.mark.parametrize("qt", [Q4_K, Q5_K])
+@pytest.mark.parametrize("TB,N,K", [(48, 1, 256), (64, 255, 256), (65, 256, 512), (96, 257, 768), (97, 31, 2304), (128, 600, 512),
+                                    (129, 33, 256), (160, 512, 1024), (257, 300, 768)])
+def test_gemm_prefill_tile_edges(miq, oracle, dev, qt, TB, N, K, switch):
+    """The fp16 GEMM at the edges of its tiles (256 rows of 32-row waves; 32, 64, 96 and
+    128 tokens), of one K block per range and of uneven ranges, with a strided output and
+    a residual: the per-output summation-order bound, nothing written beside the outputs."""
+    import torch
+    switch("PREFILL_FP16", "2")
+    wq = weights(miq, qt, N, K, seed=TB * 7 + N)
+    rng = np.random.default_rng(TB + K)
+    x = rng.standard_normal((TB, K)).astype(np.float32)
+    res = rng.standard_normal((TB, N + 3)).astype(np.float32)
+    out = torch.full((TB + 1, N + 3), 7.0, dtype=torch.float32, device=dev)
+    act = miq.xq(torch.from_numpy(x).to(dev))
+    wd, rd = torch.from_numpy(wq).to(dev), torch.from_numpy(res).to(dev)
+    miq.i8_gemm(miq.make_seg(wd, qt, K, N, act, out, N + 3, residual=rd, alpha=0.5), TB)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert (got[TB:] == 7.0).all() and (got[:, N:] == 7.0).all()
+    a = oracle.xq(x)
+    exp = 0.5 * oracle.gemm(qt, wq, K, N, a) + res[:, :N]
+    assert_elem(got[:TB, :N], exp, elem_bound(oracle, qt, wq, K, a, 0.5), residual=res[:, :N])
+
+
+@pytest.mark.parametrize("TB,K,rows", [(77, 512, (300, 256, 17)), (200, 768, (1024, 40)), (512, 256, (2048, 4352))])
+def test_quant_gemm_multi_prefill(miq, dev, TB, K, rows, switch):
+    """Several matrices in one prefill launch, each with its own schedule: every
+    segment's outputs equal its own call's bit for bit."""
+    import torch
+    switch("PREFILL_FP16", "2")
+    x = torch.from_numpy(np.random.default_rng(TB).standard_normal((TB, K)).astype(np.float32)).to(dev)
+    ws = [torch.from_numpy(weights(miq, Q4_K, n, K, seed=n)).to(dev) for n in rows]
+    outs = [[torch.full((TB, n), float("nan"), device=dev) for n in rows] for _ in range(2)]
+    act = miq.alloc_act(TB, K, dev)
+    segs = [[miq.make_seg(w, Q4_K, K, n, act, o, n, x=x, alpha=1.0 + i) for i, (w, n, o) in enumerate(zip(ws, rows, os))]
+            for os in outs]
+    for _ in range(2):
+        miq.quant_gemm_multi(segs[0], TB)
+    for s in segs[1]:
+        miq.quant_gemm(s, TB)
+    torch.cuda.synchronize()
+    for a, b in zip(*outs):
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
 def test_gemm_prefill_fp16_stream_k(miq, oracle, dev, switch):
     """512 x 16640: 520 tiles of 128 x 128 on 512 resident workgroups, so every
     tile's K blocks are dealt out as contiguous ranges (stream-K), partial sums
