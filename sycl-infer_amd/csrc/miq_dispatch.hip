@@ -26,7 +26,8 @@ Route route(const miq_seg *s, int TB) {
     // 16-token kernel, 2 the fp16 GEMM at every prefill size, 0 the int8
     // tiled kernel instead (A/B switches)
     const int pf_mode = sw(kSwPrefillFp16);
-    const bool pf16 = pf_mode == 2 || (pf_mode == 1 && pf16_serves(s) && (pfr_serves(s) && !static_scratch_mode() ? pfr_prefers(s, TB) : pf16_prefers(s, TB)));
+    const bool pf16 = pf_mode == 2 || (pf_mode == 1 && pf16_serves(s) &&
+                                       (static_scratch_mode() ? pf16_refuses_noalloc(s, TB) : pf16_prefers(s, TB)));
     if (TB >= min_tb32 && pf16 && pf16_serves(s)) return kRoutePf16;
     if (TB >= min_tb32 && (pf_mode == 0 || !pf16_serves(s)) && mfma32_serves(s) && mfma32_fills(s, TB))
         return kRouteM32;
@@ -41,10 +42,10 @@ int run_gemm(hipStream_t stream, const miq_seg *s, int TB, const char *who) {
     switch (route(s, TB)) {
     case kRouteGemv: return launch_gemv(stream, s, TB);
     case kRoutePf16: {
-        const int rc = pfr_serves(s) ? launch_pfr(stream, s, 1, TB) : launch_pf16(stream, s, TB);
-        // no workspace (the stream captures a graph, and this shape was not run
-        // before): a batch below the size that always needed one still runs
-        if (rc == MIQ_UNSUPPORTED && sw(kSwPrefillFp16) == 1 && !pf16_prefers(s, TB) && mfma16_fits(s)) return launch_mfma16(stream, s, TB);
+        const int rc = launch_pf16(stream, s, 1, TB);
+        // no workspace (the stream captures a graph and this shape was not run before)
+        if (rc == MIQ_UNSUPPORTED && sw(kSwPrefillFp16) == 1 && !pf16_refuses_noalloc(s, TB) && mfma16_fits(s))
+            return launch_mfma16(stream, s, TB);
         return rc;
     }
     case kRouteM32: return launch_mfma32(stream, s, TB);
@@ -57,15 +58,16 @@ int run_gemm(hipStream_t stream, const miq_seg *s, int TB, const char *who) {
 }
 
 // Segments of one activation past the GEMV's batch sizes: one launch of the
-// split-K 16-token kernel when every segment goes there, else one call each.
+// split-K 16-token kernel or of the fp16 GEMM when every segment goes there,
+// else one call each.
 int run_gemm_multi(hipStream_t stream, const miq_seg *s, int n_segs, int TB, bool one_type, const char *who) {
     bool m16 = one_type;
     for (int i = 0; m16 && i < n_segs; i++) m16 = route(&s[i], TB) == kRouteM16;
     if (m16) return launch_mfma16_multi(stream, s, n_segs, TB);
-    bool pfr = one_type && pfr_serves(s);
-    for (int i = 0; pfr && i < n_segs; i++) pfr = route(&s[i], TB) == kRoutePf16;
-    if (pfr) {
-        const int rc = launch_pfr(stream, s, n_segs, TB);
+    bool pf16 = one_type;
+    for (int i = 0; pf16 && i < n_segs; i++) pf16 = route(&s[i], TB) == kRoutePf16;
+    if (pf16) {
+        const int rc = launch_pf16(stream, s, n_segs, TB);
         if (rc != MIQ_UNSUPPORTED) return rc;
     }
     for (int i = 0; i < n_segs; i++)
@@ -186,7 +188,7 @@ int miq_group_dots(hipStream_t stream, const void *w, uint32_t type, int K, int 
     // paths 1 and 4 both name the 16-token kernels' decoders (the split-K
     // and CU-resident forms share one per type)
     if (path == 1 || path == 4) return miq::launch_mfma16_dots(stream, &s, TB, out);
-    if (path == 2) return miq::pfr_serves(&s) ? miq::launch_pfr_dots(stream, &s, TB, out) : miq::launch_pf16_dots(stream, &s, TB, out);
+    if (path == 2) return miq::launch_pf16_dots(stream, &s, TB, out);
     if (path == 5) return miq::launch_piece_dots(stream, &s, TB, out);
     if (path == 3) {
         if (!miq::mfma32_serves(&s)) {

@@ -53,16 +53,13 @@ bool mfma32_serves(const miq_seg *s);
 bool mfma32_fills(const miq_seg *s, int TB);
 int launch_mfma32(hipStream_t stream, const miq_seg *s, int TB, int32_t *dots = nullptr);
 
-// fp16-MFMA exact prefill GEMM (Q4_K, Q5_K)
+// fp16-MFMA exact prefill GEMM (Q4_K, Q5_K, Q6_K), every segment in one launch:
+// same type and K, one shared activation (segs[0]'s)
 bool pf16_serves(const miq_seg *s);
 bool pf16_prefers(const miq_seg *s, int TB);
-int launch_pf16(hipStream_t stream, const miq_seg *s, int TB);
-bool pfr_serves(const miq_seg *s);
-bool pfr_prefers(const miq_seg *s, int TB);
-int launch_pfr(hipStream_t stream, const miq_seg *segs, int n_segs, int TB);
-int launch_pfr_dots(hipStream_t stream, const miq_seg *s, int TB, int32_t *out);
+bool pf16_refuses_noalloc(const miq_seg *s, int TB);
+int launch_pf16(hipStream_t stream, const miq_seg *segs, int n_segs, int TB);
 int launch_pf16_dots(hipStream_t stream, const miq_seg *s, int TB, int32_t *out);
-
 
 // Q8_0 rows of any whole number of 32-value groups (the kernels above walk
 // 64-value units: K % 64 == 32 comes here); dots != nullptr: the parity form

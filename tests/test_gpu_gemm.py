@@ -411,7 +411,7 @@ def test_gemm_cu_form_default_many_tiles(miq, oracle, dev):
     assert_elem(out, exp, elem_bound(oracle, Q6_K, wq, K, act, 1.0), residual=None)
 
 
-@pytest.mark.parametrize("qt", [Q4_K, Q5_K])
+@pytest.mark.parametrize("qt", [Q4_K, Q5_K, Q6_K])
 @pytest.mark.parametrize("TB,N,K", [(48, 1, 256), (64, 255, 256), (65, 256, 512), (96, 257, 768), (97, 31, 2304), (128, 600, 512),
                                     (129, 33, 256), (160, 512, 1024), (257, 300, 768)])
 def test_gemm_prefill_tile_edges(miq, oracle, dev, qt, TB, N, K, switch):
