@@ -75,6 +75,24 @@ int run_gemm_multi(hipStream_t stream, const miq_seg *s, int n_segs, int TB, boo
     return MIQ_OK;
 }
 
+// Quantize the (shared) activation and run every segment past the GEMV's batch
+// sizes: where all go to the fp16 GEMM its pre-pass quantizes, else (also when
+// it has no workspace) the quantizer's launch and then the segments.
+int run_quant_gemm(hipStream_t stream, const miq_seg *s, int n_segs, int TB, bool one_type, const char *who) {
+    if (const int rc = check_xq(s->x, s->act_up, s->x_stride, s->x_stride, s->x8, s->xmeta, s->xsumq, TB, s->K, 0)) return rc;
+    bool pf16 = one_type;
+    for (int i = 0; pf16 && i < n_segs; i++) pf16 = route(&s[i], TB) == kRoutePf16;
+    if (pf16) {
+        const int rc = launch_pf16(stream, s, n_segs, TB, true);
+        if (rc != MIQ_UNSUPPORTED) return rc;
+    }
+    const int q = launch_xq(stream, s->x, s->act_up, s->x_stride, s->x_stride, const_cast<int8_t *>(s->x8),
+                            const_cast<float *>(s->xmeta), const_cast<int32_t *>(s->xsumq), TB, s->K);
+    if (q != MIQ_OK) return q;
+    if (one_type && TB <= sw(kSwGemvMaxTb) && gemv_fits(s, TB)) return launch_gemv_multi(stream, s, n_segs, TB);
+    return run_gemm_multi(stream, s, n_segs, TB, one_type, who);
+}
+
 }  // namespace miq
 
 extern "C" {
@@ -96,11 +114,7 @@ int miq_quant_gemm(hipStream_t stream, const miq_seg *seg, int TB) {
     // reference's i8_grp_quant_gemv_launch, kernels.h:216-236)
     const int gemv_max = miq::sw(miq::kSwGemvMaxTb);
     if (miq::sw(miq::kSwFusedQuant) && TB <= gemv_max && miq::gemv_quant_fits(seg, TB)) return miq::launch_gemv(stream, seg, TB, true);
-    const int q = miq::launch_xq(stream, seg->x, seg->act_up, seg->x_stride, seg->x_stride,
-                                 const_cast<int8_t *>(seg->x8), const_cast<float *>(seg->xmeta),
-                                 const_cast<int32_t *>(seg->xsumq), TB, seg->K);
-    if (q != MIQ_OK) return q;
-    return miq::run_gemm(stream, seg, TB, "miq_quant_gemm");
+    return miq::run_quant_gemm(stream, seg, 1, TB, true, "miq_quant_gemm");
 }
 
 namespace {
@@ -150,13 +164,7 @@ int miq_quant_gemm_multi(hipStream_t stream, const miq_seg *segs, int n_segs, in
     }
     if (one && miq::sw(miq::kSwFusedQuant) && TB <= miq::sw(miq::kSwGemvMaxTb) && miq::gemv_quant_fits(&s[0], TB))
         return miq::launch_gemv_multi(stream, s, n_segs, TB, true);
-    const int q = miq::launch_xq(stream, s[0].x, s[0].act_up, s[0].x_stride, s[0].x_stride,
-                                 const_cast<int8_t *>(s[0].x8), const_cast<float *>(s[0].xmeta),
-                                 const_cast<int32_t *>(s[0].xsumq), TB, s[0].K);
-    if (q != MIQ_OK) return q;
-    if (one && TB <= miq::sw(miq::kSwGemvMaxTb) && miq::gemv_fits(&s[0], TB))
-        return miq::launch_gemv_multi(stream, s, n_segs, TB);
-    return miq::run_gemm_multi(stream, s, n_segs, TB, one, "miq_quant_gemm_multi");
+    return miq::run_quant_gemm(stream, s, n_segs, TB, one, "miq_quant_gemm_multi");
 }
 
 int miq_group_dots(hipStream_t stream, const void *w, uint32_t type, int K, int n_rows, const int8_t *x8,

@@ -27,6 +27,9 @@ int sw(Switch s);
 int device_cus(int *n);
 
 int check_seg(const miq_seg *s, int TB, const char *who);
+// launch_xq's argument checks alone
+int check_xq(const float *x, const float *up, int x_stride, int up_stride, const int8_t *x8, const float *xmeta,
+             const int32_t *xsumq, int TB, int K, int layout);
 int launch_xq(hipStream_t stream, const float *x, const float *up, int x_stride, int up_stride, int8_t *x8,
               float *xmeta, int32_t *xsumq, int TB, int K, int layout = 0);
 
@@ -58,7 +61,8 @@ int launch_mfma32(hipStream_t stream, const miq_seg *s, int TB, int32_t *dots = 
 bool pf16_serves(const miq_seg *s);
 bool pf16_prefers(const miq_seg *s, int TB);
 bool pf16_refuses_noalloc(const miq_seg *s, int TB);
-int launch_pf16(hipStream_t stream, const miq_seg *segs, int n_segs, int TB);
+// quant: segs[0]'s x (and act_up) is quantized into its x8/xmeta/xsumq first, in the pre-pass
+int launch_pf16(hipStream_t stream, const miq_seg *segs, int n_segs, int TB, bool quant = false);
 int launch_pf16_dots(hipStream_t stream, const miq_seg *s, int TB, int32_t *out);
 
 // Q8_0 rows of any whole number of 32-value groups (the kernels above walk

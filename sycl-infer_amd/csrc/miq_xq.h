@@ -112,6 +112,42 @@ __device__ __forceinline__ void xq_one(const float *__restrict__ x, const float 
     }
 }
 
+// Eight consecutive lanes hold a group, lane l (= lane id & 7) its values
+// 4l..4l+3: the lane's four codes as one dword, the code sums (sq: lanes 0..3
+// s0, lanes 4..7 s1; s1 in lane 0) and the group's scale.  Max and integer
+// sums do not depend on the order, and every per-value step is xq_one's, so
+// the bytes equal xq_one's.
+__device__ __forceinline__ void xq_lane4(const float (&v)[4], uint32_t &word, int &sq, int &s1, float &sc) {
+    float mx = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float a = fabsf(v[i]);
+        mx = mx < a ? a : mx;
+    }
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) {
+        const float b = __shfl_xor(mx, o, 64);
+        mx = mx < b ? b : mx;
+    }
+    const float inv = mx > 0.0f ? 127.0f / mx : 0.0f;
+    sq = 0;
+    word = 0;
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+        float r = roundf(v[b] * inv);
+        r = r < 127.0f ? r : 127.0f;
+        r = -127.0f > r ? -127.0f : r;
+        const int q = (int)r;
+        sq += q;
+        word |= ((uint32_t)q & 0xFFu) << (8 * b);
+    }
+    sq += __shfl_xor(sq, 1, 64);
+    sq += __shfl_xor(sq, 2, 64);            // lanes 0..3: s0, lanes 4..7: s1
+    s1 = __shfl_xor(sq, 4, 64);  // lane 0: s1
+    const float scale = mx > 0.0f ? mx / 127.0f : 0.0f;
+    sc = h2f(f2h_trunc(scale));
+}
+
 // The same quantizer with eight lanes per (token, group): lane l = gid8 & 7
 // holds values 4l..4l+3 (one 16-byte load of x, and of up), the group's max
 // and the two code sums meet across the eight lanes, and each lane stores its
@@ -140,35 +176,11 @@ __device__ __forceinline__ void xq_lanes(const float *__restrict__ x, const floa
             v[3] = silu(v[3]) * b.w;
         }
     }
-    float mx = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const float a = fabsf(v[i]);
-        mx = mx < a ? a : mx;
-    }
-#pragma unroll
-    for (int o = 1; o < 8; o <<= 1) {
-        const float b = __shfl_xor(mx, o, 64);
-        mx = mx < b ? b : mx;
-    }
-    const float inv = mx > 0.0f ? 127.0f / mx : 0.0f;
-    int sq = 0;
-    uint32_t word = 0;
-#pragma unroll
-    for (int b = 0; b < 4; b++) {
-        float r = roundf(v[b] * inv);
-        r = r < 127.0f ? r : 127.0f;
-        r = -127.0f > r ? -127.0f : r;
-        const int q = (int)r;
-        sq += q;
-        word |= ((uint32_t)q & 0xFFu) << (8 * b);
-    }
-    sq += __shfl_xor(sq, 1, 64);
-    sq += __shfl_xor(sq, 2, 64);            // lanes 0..3: s0, lanes 4..7: s1
-    const int s1 = __shfl_xor(sq, 4, 64);  // lane 0: s1
+    uint32_t word;
+    int sq, s1;
+    float sc;
+    xq_lane4(v, word, sq, s1, sc);
     if (!live) return;
-    const float scale = mx > 0.0f ? mx / 127.0f : 0.0f;
-    const float sc = h2f(f2h_trunc(scale));
     if constexpr (LAYOUT == 0) {
         const size_t gi = (size_t)g * TB + t;
         reinterpret_cast<uint32_t *>(x8 + gi * 32)[l] = word;

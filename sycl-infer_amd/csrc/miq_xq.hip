@@ -18,8 +18,8 @@ __global__ __launch_bounds__(256) void expf_range_kernel(uint32_t first, uint32_
     if (i < count) y[i] = expf_libm(__builtin_bit_cast(float, first + i));
 }
 
-int launch_xq(hipStream_t stream, const float *x, const float *up, int x_stride, int up_stride, int8_t *x8,
-              float *xmeta, int32_t *xsumq, int TB, int K, int layout) {
+int check_xq(const float *x, const float *up, int x_stride, int up_stride, const int8_t *x8, const float *xmeta,
+             const int32_t *xsumq, int TB, int K, int layout) {
     if (!x || !x8 || !xmeta || (!xsumq && layout == 0) || TB <= 0 || K <= 0 || K % (layout ? 64 : 32) ||
         x_stride < K || (up && up_stride < K) || layout < 0 || layout > 2 || (layout == 2 && K % 256)) {
         set_error("miq_xq: bad arguments (TB=%d K=%d x_stride=%d)", TB, K, x_stride);
@@ -30,12 +30,18 @@ int launch_xq(hipStream_t stream, const float *x, const float *up, int x_stride,
         set_error("miq_xq: misaligned buffers (x/up 16 B with strides %% 4, x8 16 B, xmeta/xsumq 8 B)");
         return MIQ_UNSUPPORTED;
     }
-    const int G = K / 32;
-    const long n8 = (long)TB * G * 8;  // eight lanes per (token, group)
-    if (n8 >= (1L << 31)) {
-        set_error("miq_xq: %d tokens x %d groups is too large", TB, G);
+    if ((long)TB * (K / 32) * 8 >= (1L << 31)) {
+        set_error("miq_xq: %d tokens x %d groups is too large", TB, K / 32);
         return MIQ_UNSUPPORTED;
     }
+    return MIQ_OK;
+}
+
+int launch_xq(hipStream_t stream, const float *x, const float *up, int x_stride, int up_stride, int8_t *x8,
+              float *xmeta, int32_t *xsumq, int TB, int K, int layout) {
+    if (const int rc = check_xq(x, up, x_stride, up_stride, x8, xmeta, xsumq, TB, K, layout)) return rc;
+    const int G = K / 32;
+    const long n8 = (long)TB * G * 8;  // eight lanes per (token, group)
     const dim3 grid((unsigned)((n8 + 255) / 256)), block(256);
     if (layout == 0)
         hipLaunchKernelGGL(xq_kernel<0>, grid, block, 0, stream, x, up, x_stride, up_stride, x8, xmeta, xsumq, TB, G);
