@@ -69,7 +69,7 @@ constexpr int kPfRing = 3;    // activation stages in LDS
 //   U   [TT][64 lanes][16 B]            bf16 terms of sx*xsum: lane (li, lq) term
 //       lq (hi, mid, lo, 0) of the eight groups
 constexpr size_t pf_x_bytes(int TT) { return (size_t)8 * TT * 1024; }
-constexpr size_t pf_aux_bytes(int TT) { return (size_t)TT * 512 + (size_t)TT * 1024; }
+constexpr size_t pf_aux_bytes(int TT) { return ((size_t)TT * 512 + (size_t)TT * 1024 + 1023) / 1024 * 1024; }
 constexpr size_t pf_rec_bytes(int TT) { return pf_x_bytes(TT) + pf_aux_bytes(TT); }
 constexpr int pf_lds_bytes(int TT) { return kPfRing * 4 * TT * 1024 + 2 * (int)pf_aux_bytes(TT) + kPN * 8; }
 
@@ -484,10 +484,9 @@ __global__ __launch_bounds__(kPT, 2) void pf16_kernel(PfArgs A) {
     constexpr int kAux = (int)pf_aux_bytes(TT);
     constexpr int kLAux = kPfRing * kStage;              // aux, two blocks
     constexpr int kLD = kLAux + 2 * kAux;                // [wave][row tile][d, dmin][16]
-    constexpr int kXn = 4 * TT / kPW;                    // X DMA instructions per wave and stage
+    constexpr int kXn = (4 * TT + kPW - 1) / kPW;        // X DMA instructions per wave and stage (the last may be idle)
     constexpr int kAn = (kAux / 1024 + kPW - 1) / kPW;   // aux DMA instructions per wave (the last may be idle)
     constexpr int kRl = 2 * pf_raw_loads<TYPE>();
-    static_assert(4 * TT % kPW == 0, "a stage's X splits evenly over the waves");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lq = lane >> 4;
     const int K = A.K, nkb = K / 256;
@@ -525,8 +524,9 @@ __global__ __launch_bounds__(kPT, 2) void pf16_kernel(PfArgs A) {
         auto load_x = [&](int i, int s) {
             const int sc = s < s1 ? s : s1 - 1;
             const uint32_t so = (uint32_t)(sc >> 1) * (uint32_t)pf_rec_bytes(TT) + (uint32_t)(sc & 1) * kStage;
-            const uint32_t c = (uint32_t)(wave * kXn + i) * 1024;
-            pf_dma(rr, lbase + slot + c, voff, so + c);
+            int p = wave * kXn + i;
+            if (p >= 4 * TT) p = 0;  // no piece left (odd TT): one that is fetched anyway
+            pf_dma(rr, lbase + slot + p * 1024, voff, so + p * 1024);
             if (i == kXn - 1) slot = slot == (kPfRing - 1) * kStage ? 0 : slot + kStage;
         };
         auto load_aux = [&](int i, int kb) {
@@ -587,13 +587,18 @@ __global__ __launch_bounds__(kPT, 2) void pf16_kernel(PfArgs A) {
                 };
                 auto read_sx = [&](auto gl_c) {
                     constexpr int gl = decltype(gl_c)::value;
-                    using V = std::conditional_t<TT % 4 == 0, f4, f2>;
-                    constexpr int n = sizeof(V) / 4;
-                    const V *p = reinterpret_cast<const V *>(aux + ((4 * hf + gl) * 16 + li) * TT * 4);
+                    const float *p = reinterpret_cast<const float *>(aux) + ((4 * hf + gl) * 16 + li) * TT;
+                    if constexpr (TT % 2) {
 #pragma unroll
-                    for (int i = 0; i < TT / n; i++)
+                        for (int i = 0; i < TT; i++) sx[gl & 1][i] = p[i];
+                    } else {
+                        using V = std::conditional_t<TT % 4 == 0, f4, f2>;
+                        constexpr int n = sizeof(V) / 4;
 #pragma unroll
-                        for (int v = 0; v < n; v++) sx[gl & 1][n * i + v] = p[i][v];
+                        for (int i = 0; i < TT / n; i++)
+#pragma unroll
+                            for (int v = 0; v < n; v++) sx[gl & 1][n * i + v] = reinterpret_cast<const V *>(p)[i][v];
+                    }
                 };
                 read_x(std::integral_constant<int, 0>{});
                 read_x(std::integral_constant<int, 1>{});
@@ -875,16 +880,29 @@ template <int TT> static const void *pf_fn(uint32_t type, bool dots) {
     return dots ? (const void *)pf16_kernel<MIQ_TYPE_Q6_K, TT, true> : (const void *)pf16_kernel<MIQ_TYPE_Q6_K, TT>;
 }
 static const void *pf_fn(uint32_t type, int TT, bool dots) {
-    return TT == 2 ? pf_fn<2>(type, dots) : TT == 4 ? pf_fn<4>(type, dots) : TT == 6 ? pf_fn<6>(type, dots) : pf_fn<8>(type, dots);
+    switch (TT) {
+    case 2: return pf_fn<2>(type, dots);
+    case 3: return pf_fn<3>(type, dots);
+    case 4: return pf_fn<4>(type, dots);
+    case 5: return pf_fn<5>(type, dots);
+    case 6: return pf_fn<6>(type, dots);
+    case 7: return pf_fn<7>(type, dots);
+    default: return pf_fn<8>(type, dots);
+    }
 }
-static const void *pf_prep_fn(int TT) {
-    return TT == 2 ? (const void *)pf_prep_kernel<2> : TT == 4 ? (const void *)pf_prep_kernel<4>
-         : TT == 6 ? (const void *)pf_prep_kernel<6> : (const void *)pf_prep_kernel<8>;
+template <int TT> static const void *pf_pre_fn(bool quant) {
+    return quant ? (const void *)pf_quant_kernel<TT> : (const void *)pf_prep_kernel<TT>;
 }
-
-static const void *pf_quant_fn(int TT) {
-    return TT == 2 ? (const void *)pf_quant_kernel<2> : TT == 4 ? (const void *)pf_quant_kernel<4>
-         : TT == 6 ? (const void *)pf_quant_kernel<6> : (const void *)pf_quant_kernel<8>;
+static const void *pf_pre_fn(int TT, bool quant) {
+    switch (TT) {
+    case 2: return pf_pre_fn<2>(quant);
+    case 3: return pf_pre_fn<3>(quant);
+    case 4: return pf_pre_fn<4>(quant);
+    case 5: return pf_pre_fn<5>(quant);
+    case 6: return pf_pre_fn<6>(quant);
+    case 7: return pf_pre_fn<7>(quant);
+    default: return pf_pre_fn<8>(quant);
+    }
 }
 
 // more than 64 KiB of dynamic LDS (TT = 8)
@@ -897,7 +915,7 @@ static int pf_lds_limit() {
     }
     if (!lds_set[dev]) {
         for (uint32_t type : {MIQ_TYPE_Q4_K, MIQ_TYPE_Q5_K, MIQ_TYPE_Q6_K})
-            for (int TT : {2, 4, 6, 8})
+            for (int TT = 2; TT <= 8; TT++)
                 for (bool dots : {false, true})
                     if (hipFuncSetAttribute(pf_fn(type, TT, dots), hipFuncAttributeMaxDynamicSharedMemorySize, pf_lds_bytes(TT)) != hipSuccess) {
                         set_error("miq prefill: cannot raise the LDS limit to %d bytes", pf_lds_bytes(TT));
@@ -914,7 +932,7 @@ bool pf16_serves(const miq_seg *s) { return s->type == MIQ_TYPE_Q4_K || s->type 
 static int pf_tile(int TB, int *mt) {
     *mt = (TB + 127) / 128;
     const int per = (TB + *mt - 1) / *mt;
-    return 2 * ((per + 31) / 32);
+    return per <= 32 ? 2 : (per + 15) / 16;
 }
 
 // This GEMM against the split-K 16-token kernel, by a model of measured times
@@ -1029,11 +1047,11 @@ static int launch(hipStream_t stream, const miq_seg *segs, int n_segs, int TB, i
     hipError_t e;
     if (quant) {
         void *pa[] = {(void *)&s->x, (void *)&s->act_up, &stride, (void *)&s->x8, (void *)&s->xmeta, (void *)&s->xsumq, &tb, &nb, &rec};
-        e = hipLaunchKernel(pf_quant_fn(TT), dim3((unsigned)(A.mt * TT * nkb)), dim3(1024), pa, 0, stream);
+        e = hipLaunchKernel(pf_pre_fn(TT, true), dim3((unsigned)(A.mt * TT * nkb)), dim3(1024), pa, 0, stream);
     } else {
         uint32_t nx = (uint32_t)(A.mt * nkb * 8 * TT * 64), na = (uint32_t)(A.mt * nkb * TT * 16);
         void *pa[] = {(void *)&s->x8, (void *)&s->xmeta, (void *)&s->xsumq, &tb, &nb, &nx, &na, &rec};
-        e = hipLaunchKernel(pf_prep_fn(TT), dim3((nx + na + 255) / 256), dim3(256), pa, 0, stream);
+        e = hipLaunchKernel(pf_pre_fn(TT, false), dim3((nx + na + 255) / 256), dim3(256), pa, 0, stream);
     }
     if (e != hipSuccess) return check_launch("miq prefill");
     void *ka[] = {&A};
