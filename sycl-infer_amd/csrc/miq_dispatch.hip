@@ -4,7 +4,8 @@
 //   TB >= 48, Q4_K/Q5_K/Q6_K               exact fp16-MFMA GEMM, stream-K schedule (miq_pf16.hip),
 //                                          where its cost model beats the 16-token kernel;
 //                                          MIQ_PREFILL_FP16=0: the int8 kernel below
-//   TB >= 48, Q8_0 (and the switch above)  LDS-tiled 32x32 int8-MFMA GEMM (miq_mfma32.hip);
+//   TB >= 48, Q8_0 (and the switch above)  LDS-tiled 32x32 int8-MFMA GEMM (miq_mfma32.hip), where its
+//                                          cost model beats the 16-token kernel;
 //                                          Q6_K only when its tiles cover every CU
 //   otherwise                              16-token int8-MFMA GEMM (miq_mfma16.hip)
 // The switch M32_MIN_TB (miq_set_switch, env MIQ_M32_MIN_TB) moves the second
@@ -29,7 +30,8 @@ Route route(const miq_seg *s, int TB) {
     const bool pf16 = pf_mode == 2 || (pf_mode == 1 && pf16_serves(s) &&
                                        (static_scratch_mode() ? pf16_refuses_noalloc(s, TB) : pf16_prefers(s, TB)));
     if (TB >= min_tb32 && pf16 && pf16_serves(s)) return kRoutePf16;
-    if (TB >= min_tb32 && (pf_mode == 0 || !pf16_serves(s)) && mfma32_serves(s) && mfma32_fills(s, TB))
+    if (TB >= min_tb32 && (pf_mode == 0 || !pf16_serves(s)) && mfma32_serves(s) && mfma32_fills(s, TB) &&
+        (pf_mode == 0 || static_scratch_mode() || mfma32_prefers(s, TB)))
         return kRouteM32;
     if (mfma16_fits(s)) return kRouteM16;
     return kRouteNone;
@@ -49,7 +51,13 @@ int run_gemm(hipStream_t stream, const miq_seg *s, int TB, const char *who) {
         return rc;
     }
     case kRouteM32: return launch_mfma32(stream, s, TB);
-    case kRouteM16: return launch_mfma16(stream, s, TB);
+    case kRouteM16: {
+        const int rc = launch_mfma16(stream, s, TB);
+        // no scratch (the stream captures a graph): Q8_0 prefill batches still run, unsliced
+        if (rc == MIQ_UNSUPPORTED && s->type == MIQ_TYPE_Q8_0 && TB >= sw(kSwM32MinTb) && mfma32_serves(s))
+            return launch_mfma32(stream, s, TB);
+        return rc;
+    }
     case kRouteQ80: return launch_q80(stream, s, TB);
     default: break;
     }
@@ -63,7 +71,10 @@ int run_gemm(hipStream_t stream, const miq_seg *s, int TB, const char *who) {
 int run_gemm_multi(hipStream_t stream, const miq_seg *s, int n_segs, int TB, bool one_type, const char *who) {
     bool m16 = one_type;
     for (int i = 0; m16 && i < n_segs; i++) m16 = route(&s[i], TB) == kRouteM16;
-    if (m16) return launch_mfma16_multi(stream, s, n_segs, TB);
+    if (m16) {
+        const int rc = launch_mfma16_multi(stream, s, n_segs, TB);
+        if (rc != MIQ_UNSUPPORTED) return rc;
+    }
     bool pf16 = one_type;
     for (int i = 0; pf16 && i < n_segs; i++) pf16 = route(&s[i], TB) == kRoutePf16;
     if (pf16) {

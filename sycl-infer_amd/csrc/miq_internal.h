@@ -54,6 +54,8 @@ bool mfma32_serves(const miq_seg *s);
 // Q6_K: the tiled kernel has no K split, so it takes a batch only when its
 // tiles cover every CU (else the split-K 16-token kernel is faster)
 bool mfma32_fills(const miq_seg *s, int TB);
+// Q8_0: whether it beats the 16-token kernel at this shape
+bool mfma32_prefers(const miq_seg *s, int TB);
 int launch_mfma32(hipStream_t stream, const miq_seg *s, int TB, int32_t *dots = nullptr);
 
 // fp16-MFMA exact prefill GEMM (Q4_K, Q5_K, Q6_K), every segment in one launch:

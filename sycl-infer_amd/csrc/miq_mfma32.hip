@@ -24,6 +24,7 @@ namespace miq {
 typedef int v4i32 __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v4f32 __attribute__((ext_vector_type(4)));
 
 constexpr int kBM = 64;   // tokens per workgroup
 constexpr int kBN = 128;  // weight rows per workgroup
@@ -46,6 +47,10 @@ struct M32Args {
     const float *residual;
     float alpha;
     int32_t *dots;  // parity form: [TB][n_rows][K/32] int32 group dots
+    int nt, T;      // row tiles, tiles
+    int S;          // K slices per tile
+    float *part;    // [tile][slice][8][256 threads][4] partial sums (S > 1)
+    uint32_t *cnt;  // [tile] arrival counters, zero between launches
 };
 
 // LDS layout of one step
@@ -230,11 +235,15 @@ template <uint32_t TYPE, bool DOTS = false>
 __global__ __launch_bounds__(256, 2) void mfma32_kernel(M32Args A) {
     extern __shared__ __align__(16) uint8_t lds_raw[];
     M32Lds &L = *reinterpret_cast<M32Lds *>(lds_raw);
-    const int n0 = blockIdx.x * kBN, t0 = blockIdx.y * kBM;
+    // Slices of one tile run on one XCD (blockIdx % 8, the dispatcher's placement):
+    // blockIdx = 8 * (tile / 8 * S + slice) + tile % 8.
+    const int bb = blockIdx.x >> 3, slice = bb % A.S, tile = bb / A.S * 8 + (blockIdx.x & 7);
+    if (tile >= A.T) return;
+    const int n0 = tile % A.nt * kBN, t0 = tile / A.nt * kBM;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wt = (wave >> 1) * 32, wn = (wave & 1) * 64;  // wave tile origin (tokens, rows)
     const int l32 = lane & 31, hk = lane >> 5;
-    const int nkb = A.K / 256;
+    const int kb0 = slice * (A.K / 256) / A.S, nkb = (slice + 1) * (A.K / 256) / A.S;
     const __amdgpu_buffer_rsrc_t rw = make_rsrc(A.w, A.w_bytes);
     const uint32_t xbytes = (uint32_t)(A.K / 32) * A.TB * 32, mbytes = (uint32_t)(A.K / 32) * A.TB * 8;
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(A.x8, xbytes);
@@ -248,8 +257,8 @@ __global__ __launch_bounds__(256, 2) void mfma32_kernel(M32Args A) {
     }
 
     M32Raw<TYPE> R;
-    m32_fetch<TYPE>(R, A, rw, rx, rm, rq, n0, t0, 0);
-    for (int kb = 0; kb < nkb; kb++) {
+    m32_fetch<TYPE>(R, A, rw, rx, rm, rq, n0, t0, kb0);
+    for (int kb = kb0; kb < nkb; kb++) {
         __syncthreads();  // the previous step's LDS reads are done
         m32_store<TYPE>(R, L, A, n0, t0);
         __syncthreads();
@@ -356,6 +365,66 @@ __global__ __launch_bounds__(256, 2) void mfma32_kernel(M32Args A) {
         }
     }
     if constexpr (DOTS) return;
+#pragma unroll
+    for (int j = 0; j < 2; j++) acc[j] -= t2[j];
+    if (A.S > 1) {
+        // The last slice of a tile to arrive adds the slices in slice order (the
+        // result does not depend on timing); one that finds every other one
+        // arrived keeps its sums in registers.  The partials meet in the XCD's
+        // L2 (stores drained before the arrival is counted, L1-bypassing
+        // loads); a workgroup on another XCD than expected (HW_REG_XCC_ID)
+        // fences and marks the counter so that the reducer fences too.
+        __shared__ int lflag;
+        constexpr uint32_t kFar = 1u << 20;
+        v4f32 *P = reinterpret_cast<v4f32 *>(A.part) + (size_t)tile * A.S * 2048 + threadIdx.x;
+        uint32_t *cnt = A.cnt + tile;
+        const bool far = (__builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 15) != (uint32_t)(blockIdx.x & 7);
+        if (threadIdx.x == 0) {
+            const uint32_t prev = __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            lflag = (prev & (kFar - 1)) == (uint32_t)(A.S - 1) ? 1 + (prev >= kFar) : 0;
+        }
+        __syncthreads();
+        int fl = __builtin_amdgcn_readfirstlane(lflag);
+        const bool own = fl;
+        if (own) {
+            if (threadIdx.x == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                P[((size_t)slice * 8 + i) * 256] = v4f32{acc[i >> 2][4 * (i & 3)], acc[i >> 2][4 * (i & 3) + 1], acc[i >> 2][4 * (i & 3) + 2], acc[i >> 2][4 * (i & 3) + 3]};
+            if (far) __threadfence();
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                const uint32_t prev = __hip_atomic_fetch_add(cnt, far ? 1u + kFar : 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const bool last = (prev & (kFar - 1)) == (uint32_t)(A.S - 1);
+                if (last) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                lflag = last ? 1 + (prev >= kFar) : 0;
+            }
+            __syncthreads();
+            fl = __builtin_amdgcn_readfirstlane(lflag);
+        }
+        if (!fl) return;
+        if (fl == 2 || far) __threadfence();
+        v16f sum[2] = {};
+        const __amdgpu_buffer_rsrc_t rp = make_rsrc(reinterpret_cast<v4f32 *>(A.part) + (size_t)tile * A.S * 2048, (uint32_t)A.S * 32768u);
+        for (int k = 0; k < A.S; k++) {
+            if (own && k == slice) {
+#pragma unroll
+                for (int j = 0; j < 2; j++) sum[j] += acc[j];
+                continue;
+            }
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const v4f32 q = __builtin_bit_cast(v4f32, __builtin_amdgcn_raw_buffer_load_b128(
+                                                              rp, (uint32_t)(((k * 8 + i) * 256 + (int)threadIdx.x) * 16), 0, 1));
+#pragma unroll
+                for (int v = 0; v < 4; v++) sum[i >> 2][4 * (i & 3) + v] += q[v];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[j] = sum[j];
+    }
     // write: C[token][row]
 #pragma unroll
     for (int j = 0; j < 2; j++) {
@@ -366,7 +435,7 @@ __global__ __launch_bounds__(256, 2) void mfma32_kernel(M32Args A) {
             const int t = t0 + wt + 8 * (v >> 2) + 4 * hk + (v & 3);
             if (t < A.TB) {
                 const size_t o = (size_t)t * A.out_stride + row;
-                float val = A.alpha * (acc[j][v] - t2[j][v]);
+                float val = A.alpha * acc[j][v];
                 if (A.residual) val += A.residual[o];
                 A.out[o] = val;
             }
@@ -388,6 +457,32 @@ bool mfma32_fills(const miq_seg *s, int TB) {
     return (long)((s->n_rows + kBN - 1) / kBN) * ((TB + kBM - 1) / kBM) >= cus;
 }
 
+// K slices per tile: as many as two workgroups per CU hold, of at least four
+// steps.  A step lasts about 3.4 us, mostly its own latency (decode, two
+// barriers), and a second workgroup on the CU makes it only 1.2 times longer:
+// 5120 x 5120 Q8_0 took 70 us at any batch from 48 to 333 tokens (40 to 240
+// tiles of 20 steps); sliced 25 us at 48, 31 at 128 and 52 at 333.
+static int m32_slices(const miq_seg *s, int TB, int n_cu) {
+    const int T = ((s->n_rows + kBN - 1) / kBN) * ((TB + kBM - 1) / kBM), nkb = s->K / 256;
+    const int S = 2 * n_cu / T, most = nkb / 4;
+    return S < 1 || most < 1 ? 1 : S < most ? S : most;
+}
+
+// Q8_0: this kernel against the split-K 16-token kernel, by a model of measured
+// times (us; 48..512 tokens, 1024 / 5120 / 17408 x 5120; NK in millions).
+// 16-token kernel 8 + 0.355 * ceil(TB / 16) * NK; this kernel 3.4 us a step,
+// 1.2 times that with two workgroups per CU, 1.63 for each 2 * n_cu tiles
+// beyond, and about 1.2 us per slice that the last one adds.
+bool mfma32_prefers(const miq_seg *s, int TB) {
+    if (s->type != MIQ_TYPE_Q8_0) return true;
+    int n_cu = 0;
+    if (device_cus(&n_cu) != MIQ_OK) n_cu = 256;
+    const int S = m32_slices(s, TB, n_cu), nkb = s->K / 256;
+    const double W = (double)((s->n_rows + kBN - 1) / kBN) * ((TB + kBM - 1) / kBM) * S;
+    const double f = W <= n_cu ? 1.0 : W <= 2 * n_cu ? 1.2 : 1.63 * W / (2 * n_cu);
+    return 6.0 + 3.4 * nkb / S * f + 1.2 * (S - 1) < 8.0 + 0.355 * ((TB + 15) / 16) * (double)s->n_rows * s->K * 1e-6;
+}
+
 int launch_mfma32(hipStream_t stream, const miq_seg *s, int TB, int32_t *dots) {
     M32Args A{};
     A.w = (const uint8_t *)s->w;
@@ -403,7 +498,15 @@ int launch_mfma32(hipStream_t stream, const miq_seg *s, int TB, int32_t *dots) {
     A.out_stride = s->out_stride;
     A.residual = s->residual;
     A.alpha = s->alpha;
-    const dim3 grid((s->n_rows + kBN - 1) / kBN, (TB + kBM - 1) / kBM);
+    A.nt = (s->n_rows + kBN - 1) / kBN;
+    A.T = A.nt * ((TB + kBM - 1) / kBM);
+    int n_cu = 0;
+    if (const int rc = device_cus(&n_cu)) return rc;
+    A.S = dots ? 1 : m32_slices(s, TB, n_cu);
+    // no scratch for the partials (the stream captures a graph and this shape was
+    // not run before, or beyond miq_i8_gemm_noalloc's array): unsliced
+    if (A.S > 1 && scratch_get(stream, (size_t)A.T * A.S * 32768, A.T, &A.part, &A.cnt) != MIQ_OK) A.S = 1;
+    const dim3 grid((unsigned)((A.T + 7) / 8 * 8 * A.S));
     const size_t lds = sizeof(M32Lds);
     A.dots = dots;
     if (dots) {  // parity form (miq_group_dots path 3)

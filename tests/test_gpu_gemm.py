@@ -436,6 +436,35 @@ def test_gemm_prefill_tile_edges(miq, oracle, dev, qt, TB, N, K, switch):
     assert_elem(got[:TB, :N], exp, elem_bound(oracle, qt, wq, K, a, 0.5), residual=res[:, :N])
 
 
+@pytest.mark.parametrize("qt", [Q8_0, Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("TB,N,K", [(48, 1, 768), (64, 128, 2048), (65, 129, 2560), (130, 300, 5376), (200, 1100, 4096)])
+def test_gemm_prefill_int8_slices(miq, oracle, dev, qt, TB, N, K, switch):
+    """The int8 tiled GEMM with its tiles' K cut into slices (1, 2, 2, 5 of uneven
+    length, 4), the last to arrive adding them in slice order: the per-output bound,
+    a strided output and a residual, nothing written beside, the same bits every run."""
+    import torch
+    switch("PREFILL_FP16", "0")
+    switch("M32_FILL", "0")
+    wq = weights(miq, qt, N, K, seed=TB * 11 + N)
+    rng = np.random.default_rng(TB + K + 1)
+    x = rng.standard_normal((TB, K)).astype(np.float32)
+    res = rng.standard_normal((TB, N + 3)).astype(np.float32)
+    act = miq.xq(torch.from_numpy(x).to(dev))
+    wd, rd = torch.from_numpy(wq).to(dev), torch.from_numpy(res).to(dev)
+    runs = []
+    for _ in range(3):
+        out = torch.full((TB + 1, N + 3), 7.0, dtype=torch.float32, device=dev)
+        miq.i8_gemm(miq.make_seg(wd, qt, K, N, act, out, N + 3, residual=rd, alpha=0.5), TB)
+        torch.cuda.synchronize()
+        runs.append(out.cpu().numpy())
+    got = runs[0]
+    assert all(np.array_equal(got.view(np.uint32), r.view(np.uint32)) for r in runs[1:])
+    assert (got[TB:] == 7.0).all() and (got[:, N:] == 7.0).all()
+    a = oracle.xq(x)
+    exp = 0.5 * oracle.gemm(qt, wq, K, N, a) + res[:, :N]
+    assert_elem(got[:TB, :N], exp, elem_bound(oracle, qt, wq, K, a, 0.5), residual=res[:, :N])
+
+
 @pytest.mark.parametrize("TB,K,rows", [(77, 512, (300, 256, 17)), (200, 768, (1024, 40)), (512, 256, (2048, 4352))])
 def test_quant_gemm_multi_prefill(miq, dev, TB, K, rows, switch):
     """Several matrices in one prefill launch, each with its own schedule: every
