@@ -1,15 +1,15 @@
 // Entry points of the GEMV/GEMM family and the kernel choice by batch size.
 //
 //   TB <= 3 (and the activation fits LDS)  dot4 GEMV (miq_gemv.hip)
-//   TB >= 48, Q4_K/Q5_K/Q6_K               exact fp16-MFMA GEMM, stream-K schedule (miq_pf16.hip),
+//   TB >= 33, Q4_K/Q5_K/Q6_K               exact fp16-MFMA GEMM, stream-K schedule (miq_pf16.hip),
 //                                          where its cost model beats the 16-token kernel;
 //                                          MIQ_PREFILL_FP16=0: the int8 kernel below
-//   TB >= 48, Q8_0 (and the switch above)  LDS-tiled 32x32 int8-MFMA GEMM (miq_mfma32.hip), where its
+//   TB >= 17, Q8_0 (and the switch above)  LDS-tiled 32x32 int8-MFMA GEMM (miq_mfma32.hip), where its
 //                                          cost model beats the 16-token kernel;
 //                                          Q6_K only when its tiles cover every CU
 //   otherwise                              16-token int8-MFMA GEMM (miq_mfma16.hip)
-// The switch M32_MIN_TB (miq_set_switch, env MIQ_M32_MIN_TB) moves the second
-// threshold.
+// The switch M32_MIN_TB (miq_set_switch, env MIQ_M32_MIN_TB; 17) moves the
+// smallest batch of both prefill kernels.
 #include "miq_internal.h"
 
 namespace miq {
@@ -27,11 +27,15 @@ Route route(const miq_seg *s, int TB) {
     // 16-token kernel, 2 the fp16 GEMM at every prefill size, 0 the int8
     // tiled kernel instead (A/B switches)
     const int pf_mode = sw(kSwPrefillFp16);
+    // Inside miq_i8_gemm_noalloc every batch below 48 tokens is the 16-token
+    // kernel's and every larger Q8_0 one the int8 GEMM's, whatever the models say.
+    const bool fixed = static_scratch_mode();
+    const int min_tb = fixed && min_tb32 < 48 ? 48 : min_tb32;
     const bool pf16 = pf_mode == 2 || (pf_mode == 1 && pf16_serves(s) &&
-                                       (static_scratch_mode() ? pf16_refuses_noalloc(s, TB) : pf16_prefers(s, TB)));
-    if (TB >= min_tb32 && pf16 && pf16_serves(s)) return kRoutePf16;
-    if (TB >= min_tb32 && (pf_mode == 0 || !pf16_serves(s)) && mfma32_serves(s) && mfma32_fills(s, TB) &&
-        (pf_mode == 0 || static_scratch_mode() || mfma32_prefers(s, TB)))
+                                       (fixed ? pf16_refuses_noalloc(s, TB) : TB > 32 && pf16_prefers(s, TB)));
+    if (TB >= min_tb && pf16 && pf16_serves(s)) return kRoutePf16;
+    if (TB >= min_tb && (pf_mode == 0 || !pf16_serves(s)) && mfma32_serves(s) && mfma32_fills(s, TB) &&
+        (pf_mode == 0 || fixed || mfma32_prefers(s, TB)))
         return kRouteM32;
     if (mfma16_fits(s)) return kRouteM16;
     return kRouteNone;
@@ -46,7 +50,7 @@ int run_gemm(hipStream_t stream, const miq_seg *s, int TB, const char *who) {
     case kRoutePf16: {
         const int rc = launch_pf16(stream, s, 1, TB);
         // no workspace (the stream captures a graph and this shape was not run before)
-        if (rc == MIQ_UNSUPPORTED && sw(kSwPrefillFp16) == 1 && !pf16_refuses_noalloc(s, TB) && mfma16_fits(s))
+        if (rc == MIQ_UNSUPPORTED && sw(kSwPrefillFp16) == 1 && (TB < 48 || !pf16_refuses_noalloc(s, TB)) && mfma16_fits(s))
             return launch_mfma16(stream, s, TB);
         return rc;
     }
