@@ -113,8 +113,8 @@ int miq_i8_gemm(hipStream_t stream, const miq_seg *seg, int TB);
  * segments.  At decode sizes (TB <= 3) segments of one type run in a single
  * launch whose workgroups are numbered across them (gate and up of an FFN
  * read as one stream); where every segment takes the split-K 16-token GEMM
- * (4..47 tokens) one launch of it covers all, each segment with the tiles
- * and K slices it has alone; otherwise one launch per segment.  Each segment's
+ * or the fp16 prefill GEMM one launch of it covers all, each segment with the
+ * tiles and K slices it has alone; otherwise one launch per segment.  Each segment's
  * outputs equal miq_i8_gemm's for it bit for bit.  Replaces
  * compute_backend::i8_row_gemv_multi (src/backend/backend.h:120-121). */
 int miq_i8_gemv_multi(hipStream_t stream, const miq_seg *segs, int n_segs, int TB);
@@ -131,9 +131,10 @@ int miq_quant_gemm_multi(hipStream_t stream, const miq_seg *segs, int n_segs, in
  * ends) instead of the grow-on-demand scratch.  No counterpart in the
  * reference: for callers that cannot allocate device memory (code under
  * graph capture that was never warmed up, tight serving loops, harnesses that
- * forbid hipMalloc).  Serves the decode and 16-token kernels (batches that the
- * dispatch gives the fp16 prefill GEMM need a workspace and return
- * MIQ_UNSUPPORTED), and
+ * forbid hipMalloc).  Serves the decode, 16-token and Q8_0 kernels: every batch
+ * below 48 tokens (there also where miq_i8_gemm takes a prefill kernel, whose
+ * sums differ in their last bits), beyond that the shapes too small for the
+ * fp16 prefill GEMM (the others need a workspace and return MIQ_UNSUPPORTED), and
  * returns MIQ_UNSUPPORTED for a shape whose partials exceed the array.  Every
  * call on one GPU shares its array: calls that overlap on one GPU race. */
 int miq_i8_gemm_noalloc(hipStream_t stream, const miq_seg *seg, int TB);

@@ -1,4 +1,4 @@
-// Batched decode GEMM for 5..47 tokens on int8 MFMA (v_mfma_i32_16x16x32_i8).
+// Batched decode GEMM for 4..32 tokens (and larger batches of small matrices) on int8 MFMA (v_mfma_i32_16x16x32_i8).
 //
 // One 32-value activation group is exactly one MFMA K step, so every MFMA
 // result is the exact int32 group dot of the reference (i8.cpp:49-57,109-118;

@@ -7,7 +7,8 @@
 // block per step.  Each step the workgroup decodes its 128 rows' Q4_K/Q5_K/
 // Q8_0 bytes once into int8 codes in LDS (plus per-(row, group) fp32 scales)
 // and copies the 128 tokens' codes and scales next to them; the next step's
-// raw bytes are fetched into registers while the current step computes.
+// raw bytes are fetched into registers while the current step computes.  A tile's
+// K range may be cut into slices on several workgroups (m32_slices).
 //
 // One MFMA K step is one 32-value group, so every MFMA result is the exact
 // int32 group dot of the reference (i8.cpp:49-57,109-118; q4exp.cpp:457-467);
