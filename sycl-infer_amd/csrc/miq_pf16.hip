@@ -539,7 +539,11 @@ __global__ __launch_bounds__(kPT, 2) void pf16_kernel(PfArgs A) {
         for (int a = 0; a < 2; a++)
 #pragma unroll
             for (int b = 0; b < TT; b++) acc[a][b] = f4{0, 0, 0, 0};
-        pf_sync<63>();  // the previous range is done with every LDS buffer
+        // The previous range is done with every LDS buffer: its reads, and the loads
+        // that it issued past its end.  A wave without a piece of its own fetches one
+        // of another wave's again (load_x, load_aux), so a late one of those loads
+        // and this range's own would meet in one place with nothing to order them.
+        pf_sync<0>();
         // in the order that the loop keeps: aux, X(s), weights, X(s + 1)
 #pragma unroll
         for (int i = 0; i < kAn; i++) load_aux(i, kb0);

@@ -436,6 +436,33 @@ def test_gemm_prefill_tile_edges(miq, oracle, dev, qt, TB, N, K, switch):
     assert_elem(got[:TB, :N], exp, elem_bound(oracle, qt, wq, K, a, 0.5), residual=res[:, :N])
 
 
+@pytest.mark.parametrize("qt,TB,N,K", [(Q4_K, 32, 76800, 256), (Q4_K, 48, 76800, 256), (Q5_K, 48, 65536, 512), (Q6_K, 64, 76800, 256),
+                                       (Q4_K, 80, 131072, 256), (Q5_K, 112, 76800, 256), (Q4_K, 200, 40000, 512)])
+def test_gemm_prefill_whole_tiles_in_a_row(miq, oracle, dev, qt, TB, N, K, switch):
+    """The fp16 GEMM where a workgroup finishes a whole tile and starts the next at
+    once (300 stream-K tiles, one or two data-parallel rounds of 256), at token
+    tiles of 2, 3, 4, 5 and 7 sixteens, whose waves without a load of their own
+    repeat another wave's: three tokens against the oracle, the same bits every run."""
+    import torch
+    print(f"prefill whole tiles qt={qt} TB={TB} N={N} K={K}", flush=True)
+    switch("PREFILL_FP16", "2")
+    switch("M32_MIN_TB", "17")
+    wq = weights(miq, qt, N, K, seed=TB + K)
+    x = np.random.default_rng(TB).standard_normal((TB, K)).astype(np.float32)
+    act = miq.xq(to_dev(x, dev))
+    wd = to_dev(wq, dev)
+    runs = []
+    for _ in range(3):
+        out = torch.full((TB, N), float("nan"), dtype=torch.float32, device=dev)
+        miq.i8_gemm(miq.make_seg(wd, qt, K, N, act, out, N), TB)
+        torch.cuda.synchronize()
+        runs.append(out)
+    assert all(torch.equal(runs[0].view(torch.int32), r.view(torch.int32)) for r in runs[1:])
+    sel = [0, TB // 2, TB - 1]
+    a = oracle.xq(x[sel])
+    assert_elem(runs[0][sel].cpu().numpy(), oracle.gemm(qt, wq, K, N, a), elem_bound(oracle, qt, wq, K, a, 1.0))
+
+
 @pytest.mark.parametrize("qt", [Q8_0, Q4_K, Q5_K, Q6_K])
 @pytest.mark.parametrize("TB,N,K", [(48, 1, 768), (64, 128, 2048), (65, 129, 2560), (130, 300, 5376), (200, 1100, 4096)])
 def test_gemm_prefill_int8_slices(miq, oracle, dev, qt, TB, N, K, switch):
