@@ -18,7 +18,11 @@
  *     runs a step eagerly before recording its decode graph,
  *     src/engine/engine.cpp:4528-4583), or call miq_i8_gemm_noalloc.  That
  *     scratch is shared by every stream of a device: calls that use it must
- *     not overlap on one device;
+ *     not overlap on one device.  Q8_0 batches of 48 tokens or more with
+ *     K % 256 == 0 may overlap on several streams: they run without scratch,
+ *     or faster with buffers of their stream's own, which the first eight
+ *     streams that make such a call get (up to 24 MiB each; not while a
+ *     stream captures a graph);
  *   - work is enqueued on the caller's stream and nothing waits on the host;
  *   - status: MIQ_OK (0); MIQ_UNSUPPORTED (1) for a shape/type the kernels do
  *     not serve, so the caller falls back exactly as the reference's `bool`

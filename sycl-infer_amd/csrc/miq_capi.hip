@@ -44,7 +44,8 @@ int check_launch(const char *what) {
 // pointing at it.  The counters are zeroed once at allocation and every kernel
 // that uses them leaves them at zero.  Launches that share a device share this
 // memory: calls that use it must not overlap on one device (one stream per
-// device, as the reference serialises engine execution).
+// device, as the reference serialises engine execution).  Calls that need none
+// of it to run have per-stream scratch instead (below).
 namespace {
 struct Scratch {
     float *part = nullptr;
@@ -150,12 +151,8 @@ static int static_scratch_get(hipStream_t stream, size_t part_bytes, size_t n_cn
     return MIQ_OK;
 }
 
-int scratch_get(hipStream_t stream, size_t part_bytes, size_t n_cnt, float **part, uint32_t **cnt) {
-    if (g_static_mode) return static_scratch_get(stream, part_bytes, n_cnt, part, cnt);
-    int dev = 0;
-    if (current_device(&dev) != MIQ_OK) return MIQ_EHIP;
-    std::lock_guard<std::mutex> lk(g_scr_mu);
-    Scratch &s = g_scr[dev];
+// s at least as large as asked (g_scr_mu held)
+static int grow_scratch(Scratch &s, hipStream_t stream, size_t part_bytes, size_t n_cnt) {
     if (s.part_bytes < part_bytes) {
         if (const int rc = may_grow(stream, "split-K scratch", s.part_bytes, part_bytes)) return rc;
         const size_t want = part_bytes + part_bytes / 2;
@@ -184,8 +181,66 @@ int scratch_get(hipStream_t stream, size_t part_bytes, size_t n_cnt, float **par
         s.cnt = nc;
         s.n_cnt = want;
     }
-    *part = s.part;
-    *cnt = s.cnt;
+    return MIQ_OK;
+}
+
+// ---- scratch of one stream (OwnScratch in miq_internal.h)
+//
+// For calls that run without scratch too, only slower, so that they may overlap
+// on several streams of a device: each of the first kOwnStreams streams that
+// make one has buffers of its own, every later one none.  A call under stream
+// capture gets none either (its graph may be replayed on any stream, beside
+// work of the one that captured it), nor does hipStreamPerThread (one handle
+// for a stream of every thread).  A handle that a new stream takes over from a
+// destroyed one takes the buffers over with it: HIP finishes a stream's work
+// before it gives the stream up.
+namespace {
+constexpr int kOwnStreams = 8;
+struct OwnSlot {
+    bool used = false;
+    hipStream_t stream = nullptr;
+    Scratch s;
+};
+OwnSlot g_own[kMaxDevices][kOwnStreams];
+thread_local bool g_own_mode = false;
+}  // namespace
+
+OwnScratch::OwnScratch(bool on) : before(g_own_mode) { g_own_mode = on; }
+OwnScratch::~OwnScratch() { g_own_mode = before; }
+
+static int own_scratch(hipStream_t stream, OwnSlot *slots, OwnSlot **out) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        st = hipStreamCaptureStatusActive;
+    }
+    OwnSlot *slot = nullptr;
+    for (int i = 0; i < kOwnStreams && !slot; i++)
+        if (!slots[i].used || slots[i].stream == stream) slot = &slots[i];
+    if (g_static_mode || stream == hipStreamPerThread || st != hipStreamCaptureStatusNone || !slot) {
+        set_error("split-K scratch: none for this stream");
+        return MIQ_UNSUPPORTED;
+    }
+    slot->used = true;
+    slot->stream = stream;
+    *out = slot;
+    return MIQ_OK;
+}
+
+int scratch_get(hipStream_t stream, size_t part_bytes, size_t n_cnt, float **part, uint32_t **cnt) {
+    if (g_static_mode && !g_own_mode) return static_scratch_get(stream, part_bytes, n_cnt, part, cnt);
+    int dev = 0;
+    if (current_device(&dev) != MIQ_OK) return MIQ_EHIP;
+    std::lock_guard<std::mutex> lk(g_scr_mu);
+    Scratch *s = &g_scr[dev];
+    if (g_own_mode) {
+        OwnSlot *slot = nullptr;
+        if (const int rc = own_scratch(stream, g_own[dev], &slot)) return rc;
+        s = &slot->s;
+    }
+    if (const int rc = grow_scratch(*s, stream, part_bytes, n_cnt)) return rc;
+    *part = s->part;
+    *cnt = s->cnt;
     return MIQ_OK;
 }
 

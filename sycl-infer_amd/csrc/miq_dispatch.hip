@@ -40,11 +40,21 @@ Route route(const miq_seg *s, int TB) {
     if (mfma16_fits(s)) return kRouteM16;
     return kRouteNone;
 }
+
+// The int8 tiled GEMM needs no scratch to run (unsliced), so its batches may
+// overlap on several streams of a device: from 48 tokens on, whichever kernel
+// then takes them, their partials are in scratch of the stream's own or there
+// are none.  Below that they share the device's scratch as the 16-token
+// kernel's batches do.
+bool own_scratch(const miq_seg *s, int TB) {
+    return TB >= 48 && !q80_any(s) && mfma32_serves(s) && (s->type == MIQ_TYPE_Q8_0 || route(s, TB) == kRouteM32);
+}
 }  // namespace
 
 int run_gemm(hipStream_t stream, const miq_seg *s, int TB, const char *who) {
     const int rc = check_seg(s, TB, who);
     if (rc != MIQ_OK) return rc;
+    const OwnScratch scope(own_scratch(s, TB));
     switch (route(s, TB)) {
     case kRouteGemv: return launch_gemv(stream, s, TB);
     case kRoutePf16: {
@@ -57,7 +67,7 @@ int run_gemm(hipStream_t stream, const miq_seg *s, int TB, const char *who) {
     case kRouteM32: return launch_mfma32(stream, s, TB);
     case kRouteM16: {
         const int rc = launch_mfma16(stream, s, TB);
-        // no scratch (the stream captures a graph): Q8_0 prefill batches still run, unsliced
+        // no scratch (the stream captures a graph, or has none of its own): Q8_0 prefill batches still run, unsliced
         if (rc == MIQ_UNSUPPORTED && s->type == MIQ_TYPE_Q8_0 && TB >= sw(kSwM32MinTb) && mfma32_serves(s))
             return launch_mfma32(stream, s, TB);
         return rc;
@@ -76,6 +86,7 @@ int run_gemm_multi(hipStream_t stream, const miq_seg *s, int n_segs, int TB, boo
     bool m16 = one_type;
     for (int i = 0; m16 && i < n_segs; i++) m16 = route(&s[i], TB) == kRouteM16;
     if (m16) {
+        const OwnScratch scope(own_scratch(s, TB));
         const int rc = launch_mfma16_multi(stream, s, n_segs, TB);
         if (rc != MIQ_UNSUPPORTED) return rc;
     }

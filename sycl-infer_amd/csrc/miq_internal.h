@@ -9,6 +9,14 @@ namespace miq {
 // only outside stream capture (MIQ_UNSUPPORTED if `stream` captures and the
 // buffers are too small).
 int scratch_get(hipStream_t stream, size_t part_bytes, size_t n_cnt, float **part, uint32_t **cnt);
+// While one with on == true lives, this thread's scratch_get() gives buffers of
+// the stream's own, or MIQ_UNSUPPORTED where there are none.
+struct OwnScratch {
+    explicit OwnScratch(bool on);
+    ~OwnScratch();
+    OwnScratch(const OwnScratch &) = delete;
+    bool before;
+};
 // Per-device workspace buffers, one per slot, grown on demand (same lifetime,
 // sharing and capture rules as the split-K scratch).  `zero`: a new
 // allocation is zero-filled (arrival counters that their users return to zero).

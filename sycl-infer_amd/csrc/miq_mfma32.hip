@@ -504,8 +504,8 @@ int launch_mfma32(hipStream_t stream, const miq_seg *s, int TB, int32_t *dots) {
     int n_cu = 0;
     if (const int rc = device_cus(&n_cu)) return rc;
     A.S = dots ? 1 : m32_slices(s, TB, n_cu);
-    // no scratch for the partials (the stream captures a graph and this shape was
-    // not run before, or beyond miq_i8_gemm_noalloc's array): unsliced
+    // no scratch for the partials (a stream that captures a graph or has none of
+    // its own, miq_i8_gemm_noalloc): unsliced
     if (A.S > 1 && scratch_get(stream, (size_t)A.T * A.S * 32768, A.T, &A.part, &A.cnt) != MIQ_OK) A.S = 1;
     const dim3 grid((unsigned)((A.T + 7) / 8 * 8 * A.S));
     const size_t lds = sizeof(M32Lds);

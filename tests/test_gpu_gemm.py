@@ -492,6 +492,47 @@ def test_gemm_prefill_int8_slices(miq, oracle, dev, qt, TB, N, K, switch):
     assert_elem(got[:TB, :N], exp, elem_bound(oracle, qt, wq, K, a, 0.5), residual=res[:, :N])
 
 
+@pytest.mark.parametrize("TB,N,K", [(200, 5120, 2560), (64, 1024, 5120)])
+def test_q80_prefill_streams_overlap(miq, oracle, dev, TB, N, K):
+    """Q8_0 prefill (K slices; a small matrix on the 16-token kernel) queued on two
+    streams at once, and a graph of it replayed beside them: every output equals
+    the call's own result alone bit for bit, and the graph's its bound."""
+    import torch
+    print(f"q8_0 streams overlap TB={TB} N={N} K={K}", flush=True)
+    rng = np.random.default_rng(TB)
+    wqs = [weights(miq, Q8_0, N, K, seed=s) for s in (1, 2)]
+    ws = [to_dev(w, dev) for w in wqs]
+    xs = [rng.standard_normal((TB, K)).astype(np.float32) for _ in range(2)]
+    acts = [miq.xq(to_dev(x, dev)) for x in xs]
+    refs, outs = [], [[], []]
+    for w, a in zip(ws, acts):
+        r = torch.full((TB, N), float("nan"), dtype=torch.float32, device=dev)
+        miq.i8_gemm(miq.make_seg(w, Q8_0, K, N, a, r, N), TB)
+        refs.append(r)
+    go = torch.empty((TB, N), dtype=torch.float32, device=dev)
+    gseg = miq.make_seg(ws[0], Q8_0, K, N, acts[0], go, N)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        miq.i8_gemm(gseg, TB)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for i in range(2):
+        outs[i] = [torch.full((TB, N), float("nan"), dtype=torch.float32, device=dev) for _ in range(20)]
+    torch.cuda.synchronize()
+    for j in range(20):
+        for i in range(2):
+            with torch.cuda.stream(streams[i]):
+                miq.i8_gemm(miq.make_seg(ws[i], Q8_0, K, N, acts[i], outs[i][j], N), TB)
+        if j % 5 == 0:
+            g.replay()
+    torch.cuda.synchronize()
+    for i in range(2):
+        for o in outs[i]:
+            assert torch.equal(o.view(torch.int32), refs[i].view(torch.int32))
+    a = oracle.xq(xs[0])
+    assert_elem(go.cpu().numpy(), oracle.gemm(Q8_0, wqs[0], K, N, a), elem_bound(oracle, Q8_0, wqs[0], K, a, 1.0))
+
+
 @pytest.mark.parametrize("TB,K,rows", [(77, 512, (300, 256, 17)), (200, 768, (1024, 40)), (512, 256, (2048, 4352))])
 def test_quant_gemm_multi_prefill(miq, dev, TB, K, rows, switch):
     """Several matrices in one prefill launch, each with its own schedule: every

@@ -1,0 +1,140 @@
+"""The host side of the GEMM entry points without a GPU: which kernels a call
+launches and which library buffers they get, on a recording stand-in for the
+HIP runtime (tests/cpp/fake_hip.cpp) -- where an allocation fails, where the
+stream captures a graph, and on several streams.  Each case runs in a process
+of its own, since libmiq.so there binds to the stand-in."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SRC = os.path.join(REPO, "tests", "cpp", "fake_hip.cpp")
+
+PRELUDE = r'''
+import ctypes, importlib.util, os, re, sys
+repo, fake_path = sys.argv[1:3]
+fake = ctypes.CDLL(fake_path, mode=ctypes.RTLD_GLOBAL)
+fake.fake_name.restype = ctypes.c_char_p
+fake.fake_buffer.restype = fake.fake_allocated.restype = ctypes.c_uint64
+fake.fake_malloc_limit.argtypes = [ctypes.c_size_t]
+spec = importlib.util.spec_from_file_location("miq_host", os.path.join(repo, "sycl-infer_amd", "__init__.py"))
+miq = importlib.util.module_from_spec(spec)
+sys.modules["miq_host"] = miq
+spec.loader.exec_module(miq)
+lib = miq.lib()
+Q8_0, Q4_K, Q5_K, Q6_K = 8, 12, 13, 14
+OK, UNSUPPORTED, EHIP = 0, 1, -2
+NO_LIMIT = 2**64 - 1
+
+def seg(qt, n, k, tb, i=0):
+    a = 0x100000000 + (i << 34)  # never read
+    s = miq.Seg()
+    s.w, s.type, s.K, s.n_rows, s.out, s.out_stride, s.alpha = a, qt, k, n, a + (1 << 32), n, 1.0
+    s.x, s.x_stride = 0x4000000000, k
+    s.x8, s.xmeta, s.xsumq = 0x4100000000, 0x4200000000, 0x4300000000
+    return s
+
+def run(fn, segs, tb, stream=0):
+    """(status, kernel names, library buffers of each launch)"""
+    fake.fake_reset()
+    segs = segs if isinstance(segs, list) else [segs]
+    f = getattr(lib, "miq_" + fn)
+    if fn.endswith("multi"):
+        rc = f(stream, (miq.Seg * len(segs))(*segs), len(segs), tb)
+    else:
+        rc = f(stream, ctypes.byref(segs[0]), tb)
+    names, bufs = [], []
+    for i in range(fake.fake_launches()):
+        name = re.search(r"miq(?:12_GLOBAL__N_1)?\d+([a-z]\w*?_kernel)", fake.fake_name(i).decode()).group(1)
+        if name != "zero_u32_kernel":  # clears new counters
+            names.append(name)
+            bufs.append([b for b in (fake.fake_buffer(i, k) for k in range(16)) if b])
+    return rc, names, bufs
+
+def sliced(n, tb):
+    """whether the last launch, of the int8 tiled GEMM, has more workgroups than tiles (of 128 rows x 64 tokens)"""
+    t = -(-n // 128) * -(-tb // 64)
+    return fake.fake_blocks(fake.fake_launches() - 1) > -(-t // 8) * 8
+'''
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", SRC,
+                    "-o", lib], check=True, capture_output=True)
+
+    def run(body, **env):
+        r = subprocess.run([sys.executable, "-c", PRELUDE + body, REPO, lib], capture_output=True, text=True, timeout=60,
+                           env={**os.environ, **env})
+        assert r.returncode == 0, r.stdout + r.stderr
+
+    return run
+
+
+def test_stand_in_records_launches(host):
+    """one token, 16 tokens and a prefill batch: the GEMV, the 16-token kernel, pre-pass and GEMM"""
+    host(r"""
+rc, names, bufs = run("i8_gemm", seg(Q4_K, 4096, 4096, 1), 1)
+assert rc == OK and len(names) == 1 and "gemv" in names[0], names
+rc, names, bufs = run("i8_gemm", seg(Q4_K, 17408, 5120, 16), 16)
+assert rc == OK and names == ["m16z_kernel"] and len(bufs[0]) == 2, (names, bufs)
+rc, names, bufs = run("quant_gemm", seg(Q4_K, 17408, 5120, 512), 512)
+assert rc == OK and names == ["pf_quant_kernel", "pf16_kernel"], (rc, names)
+rc, names, bufs = run("i8_gemm", seg(Q8_0, 5120, 5120, 333), 333)
+assert rc == OK and names == ["mfma32_kernel"] and len(bufs[0]) == 2 and sliced(5120, 333), (rc, names)
+""")
+
+
+def test_q80_prefill_scratch_is_the_streams_own(host):
+    """Q8_0 prefill from 48 tokens on, on the sliced int8 GEMM and on the 16-token kernel (small matrices): the
+    partials and counters of two streams are different buffers, those of one stream the same; a stream beyond the
+    eighth, hipStreamPerThread, a capturing stream and miq_i8_gemm_noalloc get none and run the unsliced GEMM."""
+    host(r"""
+for fn in ("i8_gemm", "quant_gemm", "i8_gemv_multi"):
+    for n, k, tb, kernel in ((5120, 5120, 333, "mfma32_kernel"), (1024, 5120, 64, "m16z_kernel")):
+        s = [seg(Q8_0, n, k, tb)] if fn != "i8_gemv_multi" else [seg(Q8_0, n, k, tb, i) for i in range(2)]
+        seen = {}
+        for stream in (0, 0x5000, 0x6000, 0x5000, 0):
+            rc, names, bufs = run(fn, s, tb, stream)
+            assert rc == OK and names[-1] == kernel and len(bufs[-1]) == 2, (fn, rc, names, bufs)
+            assert seen.setdefault(stream, bufs[-1]) == bufs[-1]
+        assert len({b for v in seen.values() for b in v}) == 6, seen
+        fake.fake_capturing(1)
+        for stream in (0x5000, 0x7000):  # warmed up before or not
+            rc, names, bufs = run(fn, s, tb, stream)
+            assert rc == OK and names[-1] == "mfma32_kernel" and not bufs[-1] and not sliced(n, tb), (fn, names, bufs)
+        fake.fake_capturing(0)
+        rc, names, bufs = run(fn, s, tb, 2)
+        assert rc == OK and names[-1] == "mfma32_kernel" and not bufs[-1] and not sliced(n, tb)
+s = seg(Q8_0, 5120, 5120, 333)
+rc, names, bufs = run("i8_gemm_noalloc", s, 333)
+assert rc == OK and names == ["mfma32_kernel"] and not sliced(5120, 333)
+got = [run("i8_gemm", s, 333, 0x10000 + 16 * i) for i in range(12)]
+own = [g[2][0] for g in got if g[2][0]]
+assert all(g[0] == OK for g in got) and len(own) == 5 and len({b[0] for b in own}) == 5, own
+""")
+
+
+def test_int8_prefill_of_k_quants_scratch_is_the_streams_own(host):
+    """PREFILL_FP16=0: the K-quants on the int8 tiled GEMM, from 48 tokens on, as Q8_0"""
+    host(r"""
+bufs = [run("i8_gemm", seg(Q4_K, 5120, 5120, 200), 200, s) for s in (0x5000, 0x6000)]
+assert all(b[0] == OK and b[1] == ["mfma32_kernel"] and len(b[2][0]) == 2 for b in bufs), bufs
+assert not set(bufs[0][2][0]) & set(bufs[1][2][0])
+""", MIQ_PREFILL_FP16="0")
+
+
+def test_q80_sixteen_token_batches_share_the_device_scratch(host):
+    """below 48 tokens Q8_0 keeps the device's scratch, also under a capture that it was warmed up for"""
+    host(r"""
+for n, k, tb, kernel in ((5120, 5120, 16, "m16z_kernel"), (5120, 5120, 40, "mfma32_kernel")):
+    s = seg(Q8_0, n, k, tb)
+    a, b = run("i8_gemm", s, tb, 0x5000), run("i8_gemm", s, tb, 0x6000)
+    fake.fake_capturing(1)
+    c = run("i8_gemm", s, tb, 0x7000)
+    fake.fake_capturing(0)
+    assert a == b == c and a[0] == OK and a[1] == [kernel] and len(a[2][0]) == 2, (a, b, c)
+""")
