@@ -86,9 +86,12 @@ int run_gemm_multi(hipStream_t stream, const miq_seg *s, int n_segs, int TB, boo
     bool m16 = one_type;
     for (int i = 0; m16 && i < n_segs; i++) m16 = route(&s[i], TB) == kRouteM16;
     if (m16) {
-        const OwnScratch scope(own_scratch(s, TB));
+        // Without scratch (the stream captures a graph) the call is refused before
+        // anything runs; only Q8_0 prefill, which needs none, goes on one by one.
+        const bool own = own_scratch(s, TB);
+        const OwnScratch scope(own);
         const int rc = launch_mfma16_multi(stream, s, n_segs, TB);
-        if (rc != MIQ_UNSUPPORTED) return rc;
+        if (rc != MIQ_UNSUPPORTED || !own) return rc;
     }
     bool pf16 = one_type;
     for (int i = 0; pf16 && i < n_segs; i++) pf16 = route(&s[i], TB) == kRoutePf16;

@@ -138,3 +138,16 @@ for n, k, tb, kernel in ((5120, 5120, 16, "m16z_kernel"), (5120, 5120, 40, "mfma
     fake.fake_capturing(0)
     assert a == b == c and a[0] == OK and a[1] == [kernel] and len(a[2][0]) == 2, (a, b, c)
 """)
+
+
+def test_refused_multi_call_runs_nothing(host):
+    """several 16-token segments under a capture whose scratch is too small for them together: refused as a whole,
+    also where it would do for the first one alone"""
+    host(r"""
+first, second = seg(Q4_K, 640, 5120, 16), seg(Q4_K, 8192, 5120, 16, 1)
+assert run("i8_gemv_multi", [first], 16)[0] == OK
+fake.fake_capturing(1)
+assert run("i8_gemv_multi", [first], 16)[0] == OK
+rc, names, bufs = run("i8_gemv_multi", [first, second], 16)
+assert rc == UNSUPPORTED and not names, (rc, names)
+""")
