@@ -151,13 +151,21 @@ static int static_scratch_get(hipStream_t stream, size_t part_bytes, size_t n_cn
     return MIQ_OK;
 }
 
+// hipMalloc whose failure leaves no error behind for a later check_launch():
+// a caller may go on with a kernel that needs less.
+static bool device_alloc(void **p, size_t bytes) {
+    if (hipMalloc(p, bytes) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+}
+
 // s at least as large as asked (g_scr_mu held)
 static int grow_scratch(Scratch &s, hipStream_t stream, size_t part_bytes, size_t n_cnt) {
     if (s.part_bytes < part_bytes) {
         if (const int rc = may_grow(stream, "split-K scratch", s.part_bytes, part_bytes)) return rc;
         const size_t want = part_bytes + part_bytes / 2;
         float *np = nullptr;
-        if (hipMalloc(&np, want) != hipSuccess) {
+        if (!device_alloc((void **)&np, want)) {
             set_error("split-K scratch: hipMalloc(%zu) failed", want);
             return MIQ_EHIP;
         }
@@ -169,7 +177,7 @@ static int grow_scratch(Scratch &s, hipStream_t stream, size_t part_bytes, size_
         if (const int rc = may_grow(stream, "split-K counters", s.n_cnt * 4, n_cnt * 4)) return rc;
         const size_t want = n_cnt + n_cnt / 2 + 64;
         uint32_t *nc = nullptr;
-        if (hipMalloc(&nc, want * sizeof(uint32_t)) != hipSuccess) {
+        if (!device_alloc((void **)&nc, want * sizeof(uint32_t))) {
             set_error("split-K scratch: counter allocation failed");
             return MIQ_EHIP;
         }
@@ -238,7 +246,7 @@ int scratch_get(hipStream_t stream, size_t part_bytes, size_t n_cnt, float **par
         if (const int rc = own_scratch(stream, g_own[dev], &slot)) return rc;
         s = &slot->s;
     }
-    if (const int rc = grow_scratch(*s, stream, part_bytes, n_cnt)) return rc;
+    if (const int rc = grow_scratch(*s, stream, part_bytes, n_cnt)) return g_own_mode ? (int)MIQ_UNSUPPORTED : rc;
     *part = s->part;
     *cnt = s->cnt;
     return MIQ_OK;
@@ -269,7 +277,7 @@ int workspace_get(hipStream_t stream, int slot, size_t bytes, void **ptr, bool z
         if (const int rc = may_grow(stream, "workspace", w.bytes, bytes)) return rc;
         const size_t want = (bytes + bytes / 4 + 3) & ~(size_t)3;
         void *np = nullptr;
-        if (hipMalloc(&np, want) != hipSuccess) {
+        if (!device_alloc(&np, want)) {
             set_error("workspace: hipMalloc(%zu) failed", want);
             return MIQ_EHIP;
         }

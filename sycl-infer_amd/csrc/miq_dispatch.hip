@@ -58,9 +58,10 @@ int run_gemm(hipStream_t stream, const miq_seg *s, int TB, const char *who) {
     switch (route(s, TB)) {
     case kRouteGemv: return launch_gemv(stream, s, TB);
     case kRoutePf16: {
-        const int rc = launch_pf16(stream, s, 1, TB);
-        // no workspace (the stream captures a graph and this shape was not run before)
-        if (rc == MIQ_UNSUPPORTED && sw(kSwPrefillFp16) == 1 && (TB < 48 || !pf16_refuses_noalloc(s, TB)) && mfma16_fits(s))
+        bool no_ws;
+        const int rc = launch_pf16(stream, s, 1, TB, false, &no_ws);
+        // no workspace: the stream captures a graph and this shape was not run before, or no memory for it
+        if ((rc == MIQ_UNSUPPORTED || no_ws) && sw(kSwPrefillFp16) == 1 && (TB < 48 || !pf16_refuses_noalloc(s, TB)) && mfma16_fits(s))
             return launch_mfma16(stream, s, TB);
         return rc;
     }
@@ -96,8 +97,9 @@ int run_gemm_multi(hipStream_t stream, const miq_seg *s, int n_segs, int TB, boo
     bool pf16 = one_type;
     for (int i = 0; pf16 && i < n_segs; i++) pf16 = route(&s[i], TB) == kRoutePf16;
     if (pf16) {
-        const int rc = launch_pf16(stream, s, n_segs, TB);
-        if (rc != MIQ_UNSUPPORTED) return rc;
+        bool no_ws;
+        const int rc = launch_pf16(stream, s, n_segs, TB, false, &no_ws);
+        if (rc != MIQ_UNSUPPORTED && !no_ws) return rc;
     }
     for (int i = 0; i < n_segs; i++)
         if (const int rc = run_gemm(stream, &s[i], TB, who)) return rc;
@@ -112,8 +114,9 @@ int run_quant_gemm(hipStream_t stream, const miq_seg *s, int n_segs, int TB, boo
     bool pf16 = one_type;
     for (int i = 0; pf16 && i < n_segs; i++) pf16 = route(&s[i], TB) == kRoutePf16;
     if (pf16) {
-        const int rc = launch_pf16(stream, s, n_segs, TB, true);
-        if (rc != MIQ_UNSUPPORTED) return rc;
+        bool no_ws;
+        const int rc = launch_pf16(stream, s, n_segs, TB, true, &no_ws);
+        if (rc != MIQ_UNSUPPORTED && !no_ws) return rc;
     }
     const int q = launch_xq(stream, s->x, s->act_up, s->x_stride, s->x_stride, const_cast<int8_t *>(s->x8),
                             const_cast<float *>(s->xmeta), const_cast<int32_t *>(s->xsumq), TB, s->K);

@@ -71,8 +71,9 @@ int launch_mfma32(hipStream_t stream, const miq_seg *s, int TB, int32_t *dots = 
 bool pf16_serves(const miq_seg *s);
 bool pf16_prefers(const miq_seg *s, int TB);
 bool pf16_refuses_noalloc(const miq_seg *s, int TB);
-// quant: segs[0]'s x (and act_up) is quantized into its x8/xmeta/xsumq first, in the pre-pass
-int launch_pf16(hipStream_t stream, const miq_seg *segs, int n_segs, int TB, bool quant = false);
+// quant: segs[0]'s x (and act_up) is quantized into its x8/xmeta/xsumq first, in the pre-pass.
+// *no_ws: it failed for want of a workspace (the stream captures, or no memory), nothing was launched
+int launch_pf16(hipStream_t stream, const miq_seg *segs, int n_segs, int TB, bool quant, bool *no_ws);
 int launch_pf16_dots(hipStream_t stream, const miq_seg *s, int TB, int32_t *out);
 
 // Q8_0 rows of any whole number of 32-value groups (the kernels above walk

@@ -61,6 +61,9 @@ constexpr int kPT = 64 * kPW;
 constexpr int kPN = 32 * kPW; // weight rows per workgroup: each wave owns 32
 constexpr int kPfSegs = 8;    // matrices of one launch
 constexpr int kPfRing = 3;    // activation stages in LDS
+// Partial sums of the matrices of one launch at most (one matrix takes up to
+// 64 MiB); more matrices go out in further launches that use the same memory.
+constexpr size_t kPfPartBytes = (size_t)256 << 20;
 
 // One activation record per (token tile of 16*TT tokens, 256-value block):
 //   X   [8 groups][TT][64 lanes][16 B]  fp16 codes in MFMA operand order: lane
@@ -983,7 +986,7 @@ bool pf16_refuses_noalloc(const miq_seg *s, int TB) {
     return a0 + ac * C + cpf * mt * nk < c16 * ((TB + 15) / 16) * nk;
 }
 
-static int launch(hipStream_t stream, const miq_seg *segs, int n_segs, int TB, int32_t *dots, bool quant) {
+static int launch(hipStream_t stream, const miq_seg *segs, int n_segs, int TB, int32_t *dots, bool quant, bool *no_ws) {
     const miq_seg *s = segs;
     const int K = s->K;
     const long nkb = K / 256;
@@ -996,15 +999,16 @@ static int launch(hipStream_t stream, const miq_seg *segs, int n_segs, int TB, i
     A.row_bytes = (uint32_t)miq_row_bytes(s->type, K);
     A.K = K;
     A.TB = TB;
-    A.nseg = n_segs;
     A.dots = dots;
     int n_cu = 0;
     if (const int rc = device_cus(&n_cu)) return rc;
     if (const int rc = pf_lds_limit()) return rc;
-    uint32_t slots = 0, tiles = 0;
-    long grid = 0;
+    PfSeg seg[kPfSegs];
+    int first[kPfSegs + 1] = {0}, n_launch = 1;  // launch l: segments [first[l], first[l + 1])
+    uint32_t slots = 0, tiles = 0, max_slots = 0, max_tiles = 0;
+    const size_t slot_bytes = (size_t)2 * TT * kPT * 16;
     for (int i = 0; i < n_segs; i++) {
-        PfSeg &g = A.seg[i];
+        PfSeg &g = seg[i];
         g.w = (const uint8_t *)segs[i].w;
         g.w_bytes = dword_span((size_t)segs[i].n_rows * A.row_bytes);
         g.out = segs[i].out;
@@ -1032,17 +1036,25 @@ static int launch(hipStream_t stream, const miq_seg *segs, int n_segs, int TB, i
         g.P = (int)P;
         g.rounds = (int)rounds;
         g.xmap = !dots && sk >= 8 && P % 8 == 0;
+        const uint32_t need = sk ? (uint32_t)(2 * P) : 0;
+        if (i > first[n_launch - 1] && (slots + need) * slot_bytes > kPfPartBytes) {
+            first[n_launch++] = i;
+            slots = tiles = 0;
+        }
         g.poff = slots;
         g.coff = tiles;
-        slots += sk ? (uint32_t)(2 * P) : 0;
+        slots += need;
         tiles += (uint32_t)T;
-        grid = P > grid ? P : grid;
+        max_slots = slots > max_slots ? slots : max_slots;
+        max_tiles = tiles > max_tiles ? tiles : max_tiles;
     }
+    first[n_launch] = n_segs;
     const size_t rec_bytes = align_up((size_t)A.mt * nkb * pf_rec_bytes(TT), 256);
-    const size_t part_bytes = (size_t)slots * 2 * TT * kPT * 16;
     void *ws = nullptr, *cw = nullptr;
-    if (const int rc = workspace_get(stream, kWsPrefill, rec_bytes + part_bytes, &ws)) return rc;
-    if (const int rc = workspace_get(stream, kWsPrefillCnt, (size_t)tiles * 4, &cw, true)) return rc;
+    *no_ws = true;
+    if (const int rc = workspace_get(stream, kWsPrefill, rec_bytes + max_slots * slot_bytes, &ws)) return rc;
+    if (const int rc = workspace_get(stream, kWsPrefillCnt, (size_t)max_tiles * 4, &cw, true)) return rc;
+    *no_ws = false;
     A.rec = reinterpret_cast<const uint8_t *>(ws);
     A.part = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(ws) + rec_bytes);
     A.cnt = reinterpret_cast<uint32_t *>(cw);
@@ -1059,13 +1071,22 @@ static int launch(hipStream_t stream, const miq_seg *segs, int n_segs, int TB, i
     }
     if (e != hipSuccess) return check_launch("miq prefill");
     void *ka[] = {&A};
-    if (hipLaunchKernel(pf_fn(s->type, TT, dots != nullptr), dim3((unsigned)grid), dim3(kPT), ka, pf_lds_bytes(TT), stream) != hipSuccess)
-        return check_launch("miq prefill");
+    for (int l = 0; l < n_launch; l++) {
+        int grid = 0;
+        A.nseg = first[l + 1] - first[l];
+        for (int i = 0; i < A.nseg; i++) {
+            A.seg[i] = seg[first[l] + i];
+            grid = A.seg[i].P > grid ? A.seg[i].P : grid;
+        }
+        if (hipLaunchKernel(pf_fn(s->type, TT, dots != nullptr), dim3((unsigned)grid), dim3(kPT), ka, pf_lds_bytes(TT), stream) != hipSuccess)
+            return check_launch("miq prefill");
+    }
     return check_launch("miq prefill");
 }
 
-int launch_pf16(hipStream_t stream, const miq_seg *segs, int n_segs, int TB, bool quant) {
-    return launch(stream, segs, n_segs, TB, nullptr, quant);
+int launch_pf16(hipStream_t stream, const miq_seg *segs, int n_segs, int TB, bool quant, bool *no_ws) {
+    *no_ws = false;
+    return launch(stream, segs, n_segs, TB, nullptr, quant, no_ws);
 }
 
 // Parity form (miq_group_dots path 2): one tile per workgroup with every
@@ -1076,7 +1097,8 @@ int launch_pf16_dots(hipStream_t stream, const miq_seg *s, int TB, int32_t *out)
         set_error("miq_group_dots: path 2 (the fp16 prefill decoder) serves Q4_K, Q5_K and Q6_K");
         return MIQ_UNSUPPORTED;
     }
-    return launch(stream, s, 1, TB, out, false);
+    bool no_ws;
+    return launch(stream, s, 1, TB, out, false, &no_ws);
 }
 
 }  // namespace miq

@@ -533,10 +533,12 @@ def test_q80_prefill_streams_overlap(miq, oracle, dev, TB, N, K):
     assert_elem(go.cpu().numpy(), oracle.gemm(Q8_0, wqs[0], K, N, a), elem_bound(oracle, Q8_0, wqs[0], K, a, 1.0))
 
 
-@pytest.mark.parametrize("TB,K,rows", [(77, 512, (300, 256, 17)), (200, 768, (1024, 40)), (512, 256, (2048, 4352))])
+@pytest.mark.parametrize("TB,K,rows", [(77, 512, (300, 256, 17)), (200, 768, (1024, 40)), (512, 256, (2048, 4352)),
+                                       (512, 2304, (2048,) * 6)])
 def test_quant_gemm_multi_prefill(miq, dev, TB, K, rows, switch):
-    """Several matrices in one prefill launch, each with its own schedule: every
-    segment's outputs equal its own call's bit for bit."""
+    """Several matrices in one prefill launch (the last case in two, for the size of
+    its partial sums), each with its own schedule: every segment's outputs equal its
+    own call's bit for bit."""
     import torch
     switch("PREFILL_FP16", "2")
     x = torch.from_numpy(np.random.default_rng(TB).standard_normal((TB, K)).astype(np.float32)).to(dev)

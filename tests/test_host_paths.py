@@ -151,3 +151,36 @@ assert run("i8_gemv_multi", [first], 16)[0] == OK
 rc, names, bufs = run("i8_gemv_multi", [first, second], 16)
 assert rc == UNSUPPORTED and not names, (rc, names)
 """)
+
+
+def test_no_memory_for_scratch(host):
+    """where an allocation fails, a call that can do with less still runs and reports no error: several prefill
+    segments one by one, a batch below 48 tokens on the 16-token kernel, Q8_0 prefill unsliced"""
+    host(r"""
+MiB = 2**20
+fake.fake_malloc_limit(1 * MiB)
+rc, names, bufs = run("i8_gemm", seg(Q8_0, 5120, 5120, 333), 333)
+assert rc == OK and names == ["mfma32_kernel"] and not bufs[0] and not sliced(5120, 333), (rc, names)
+rc, names, bufs = run("i8_gemm", seg(Q8_0, 1024, 5120, 200), 200)
+assert rc == OK and names == ["mfma32_kernel"] and not bufs[0] and not sliced(1024, 200), (rc, names)
+fake.fake_malloc_limit(28 * MiB)
+for fn in ("i8_gemm", "quant_gemm"):
+    rc, names, bufs = run(fn, seg(Q4_K, 17408, 5120, 40), 40)
+    assert rc == OK and names[-1] == "m16z_kernel", (rc, names)
+fake.fake_malloc_limit(100 * MiB)
+for fn in ("i8_gemv_multi", "quant_gemm_multi"):
+    rc, names, bufs = run(fn, [seg(Q4_K, 17408, 5120, 512, i) for i in range(3)], 512)
+    assert rc == OK and names.count("pf16_kernel") == 3, (rc, names)
+fake.fake_malloc_limit(1 * MiB)
+rc, names, bufs = run("i8_gemm", seg(Q4_K, 17408, 5120, 2048), 2048)
+assert rc == EHIP and not names, (rc, names)
+""")
+
+
+def test_prefill_workspace_is_bounded(host):
+    """eight prefill segments of 64 MiB of partial sums each: two launches over the same 256 MiB"""
+    host(r"""
+rc, names, bufs = run("quant_gemm_multi", [seg(Q4_K, 17408, 5120, 512, i) for i in range(8)], 512)
+assert rc == OK and names == ["pf_quant_kernel", "pf16_kernel", "pf16_kernel"] and bufs[1] == bufs[2], (names, bufs)
+assert fake.fake_allocated() < 1.25 * (256 + 16) * 2**20, fake.fake_allocated()
+""")
