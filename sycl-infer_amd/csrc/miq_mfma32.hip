@@ -232,19 +232,34 @@ __device__ __forceinline__ void m32_store(const M32Raw<TYPE> &R, M32Lds &L, cons
 
 // DOTS: the parity form -- every MFMA result (the exact int32 group dot)
 // goes to A.dots and nothing else is computed
-template <uint32_t TYPE, bool DOTS = false>
+// The forms: a workgroup takes a whole tile; a K slice of one; a whole tile in
+// the parity form.  The first is an instance of its own because the slices'
+// bookkeeping in its loop's registers costs 2 to 3 % (17408 x 5120 Q8_0 at 333
+// tokens 163 us, 167 with S == 1 as a run-time case of the second).
+enum M32Form { kM32Whole, kM32Sliced, kM32Dots };
+template <uint32_t TYPE, M32Form FORM>
 __global__ __launch_bounds__(256, 2) void mfma32_kernel(M32Args A) {
+    constexpr bool DOTS = FORM == kM32Dots;
     extern __shared__ __align__(16) uint8_t lds_raw[];
     M32Lds &L = *reinterpret_cast<M32Lds *>(lds_raw);
     // Slices of one tile run on one XCD (blockIdx % 8, the dispatcher's placement):
     // blockIdx = 8 * (tile / 8 * S + slice) + tile % 8.
-    const int bb = blockIdx.x >> 3, slice = bb % A.S, tile = bb / A.S * 8 + (blockIdx.x & 7);
-    if (tile >= A.T) return;
+    int slice = 0, tile = blockIdx.x;
+    if constexpr (FORM == kM32Sliced) {
+        const int bb = blockIdx.x >> 3;
+        slice = bb % A.S;
+        tile = bb / A.S * 8 + (blockIdx.x & 7);
+        if (tile >= A.T) return;
+    }
     const int n0 = tile % A.nt * kBN, t0 = tile / A.nt * kBM;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wt = (wave >> 1) * 32, wn = (wave & 1) * 64;  // wave tile origin (tokens, rows)
     const int l32 = lane & 31, hk = lane >> 5;
-    const int kb0 = slice * (A.K / 256) / A.S, nkb = (slice + 1) * (A.K / 256) / A.S;
+    int kb0 = 0, nkb = A.K / 256;
+    if constexpr (FORM == kM32Sliced) {
+        kb0 = slice * (A.K / 256) / A.S;
+        nkb = (slice + 1) * (A.K / 256) / A.S;
+    }
     const __amdgpu_buffer_rsrc_t rw = make_rsrc(A.w, A.w_bytes);
     const uint32_t xbytes = (uint32_t)(A.K / 32) * A.TB * 32, mbytes = (uint32_t)(A.K / 32) * A.TB * 8;
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(A.x8, xbytes);
@@ -368,7 +383,7 @@ __global__ __launch_bounds__(256, 2) void mfma32_kernel(M32Args A) {
     if constexpr (DOTS) return;
 #pragma unroll
     for (int j = 0; j < 2; j++) acc[j] -= t2[j];
-    if (A.S > 1) {
+    if constexpr (FORM == kM32Sliced) {
         // The last slice of a tile to arrive adds the slices in slice order (the
         // result does not depend on timing); one that finds every other one
         // arrived keeps its sums in registers.  The partials meet in the XCD's
@@ -484,6 +499,13 @@ bool mfma32_prefers(const miq_seg *s, int TB) {
     return 6.0 + 3.4 * nkb / S * f + 1.2 * (S - 1) < 8.0 + 0.355 * ((TB + 15) / 16) * (double)s->n_rows * s->K * 1e-6;
 }
 
+template <uint32_t TYPE> static void m32_start(const M32Args &A, M32Form form, dim3 grid, hipStream_t stream) {
+    constexpr size_t lds = sizeof(M32Lds);
+    if (form == kM32Sliced) hipLaunchKernelGGL((mfma32_kernel<TYPE, kM32Sliced>), grid, dim3(256), lds, stream, A);
+    else if (form == kM32Dots) hipLaunchKernelGGL((mfma32_kernel<TYPE, kM32Dots>), grid, dim3(256), lds, stream, A);
+    else hipLaunchKernelGGL((mfma32_kernel<TYPE, kM32Whole>), grid, dim3(256), lds, stream, A);
+}
+
 int launch_mfma32(hipStream_t stream, const miq_seg *s, int TB, int32_t *dots) {
     M32Args A{};
     A.w = (const uint8_t *)s->w;
@@ -507,25 +529,16 @@ int launch_mfma32(hipStream_t stream, const miq_seg *s, int TB, int32_t *dots) {
     // no scratch for the partials (a stream that captures a graph or has none of
     // its own, miq_i8_gemm_noalloc): unsliced
     if (A.S > 1 && scratch_get(stream, (size_t)A.T * A.S * 32768, A.T, &A.part, &A.cnt) != MIQ_OK) A.S = 1;
-    const dim3 grid((unsigned)((A.T + 7) / 8 * 8 * A.S));
-    const size_t lds = sizeof(M32Lds);
-    A.dots = dots;
-    if (dots) {  // parity form (miq_group_dots path 3)
-        switch (s->type) {
-        case MIQ_TYPE_Q4_K: hipLaunchKernelGGL((mfma32_kernel<MIQ_TYPE_Q4_K, true>), grid, dim3(256), lds, stream, A); break;
-        case MIQ_TYPE_Q5_K: hipLaunchKernelGGL((mfma32_kernel<MIQ_TYPE_Q5_K, true>), grid, dim3(256), lds, stream, A); break;
-        case MIQ_TYPE_Q6_K: hipLaunchKernelGGL((mfma32_kernel<MIQ_TYPE_Q6_K, true>), grid, dim3(256), lds, stream, A); break;
-        default: hipLaunchKernelGGL((mfma32_kernel<MIQ_TYPE_Q8_0, true>), grid, dim3(256), lds, stream, A); break;
-        }
-        return check_launch("miq_group_dots");
-    }
+    const M32Form form = dots ? kM32Dots : A.S > 1 ? kM32Sliced : kM32Whole;
+    const dim3 grid((unsigned)(form == kM32Sliced ? (A.T + 7) / 8 * 8 * A.S : A.T));
+    A.dots = dots;  // the parity form is miq_group_dots path 3
     switch (s->type) {
-    case MIQ_TYPE_Q4_K: hipLaunchKernelGGL(mfma32_kernel<MIQ_TYPE_Q4_K>, grid, dim3(256), lds, stream, A); break;
-    case MIQ_TYPE_Q5_K: hipLaunchKernelGGL(mfma32_kernel<MIQ_TYPE_Q5_K>, grid, dim3(256), lds, stream, A); break;
-    case MIQ_TYPE_Q6_K: hipLaunchKernelGGL(mfma32_kernel<MIQ_TYPE_Q6_K>, grid, dim3(256), lds, stream, A); break;
-    default: hipLaunchKernelGGL(mfma32_kernel<MIQ_TYPE_Q8_0>, grid, dim3(256), lds, stream, A); break;
+    case MIQ_TYPE_Q4_K: m32_start<MIQ_TYPE_Q4_K>(A, form, grid, stream); break;
+    case MIQ_TYPE_Q5_K: m32_start<MIQ_TYPE_Q5_K>(A, form, grid, stream); break;
+    case MIQ_TYPE_Q6_K: m32_start<MIQ_TYPE_Q6_K>(A, form, grid, stream); break;
+    default: m32_start<MIQ_TYPE_Q8_0>(A, form, grid, stream); break;
     }
-    return check_launch("miq mfma32");
+    return check_launch(dots ? "miq_group_dots" : "miq mfma32");
 }
 
 }  // namespace miq

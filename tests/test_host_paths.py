@@ -184,3 +184,16 @@ rc, names, bufs = run("quant_gemm_multi", [seg(Q4_K, 17408, 5120, 512, i) for i 
 assert rc == OK and names == ["pf_quant_kernel", "pf16_kernel", "pf16_kernel"] and bufs[1] == bufs[2], (names, bufs)
 assert fake.fake_allocated() < 1.25 * (256 + 16) * 2**20, fake.fake_allocated()
 """)
+
+
+def test_int8_prefill_forms(host):
+    """the int8 tiled GEMM's instance without slices (one workgroup per tile) wherever a tile is not cut, else the
+    sliced one (eight tiles' slices at a time)"""
+    host(r"""
+form = lambda: re.search(r"M32FormE(\d)", fake.fake_name(fake.fake_launches() - 1).decode()).group(1)
+for n, k, tb, s in ((17408, 5120, 333, 1), (5120, 5120, 512, 1), (5120, 512, 100, 1), (5120, 5120, 333, 2), (5120, 5120, 48, 5)):
+    rc, names, _ = run("i8_gemm", seg(Q8_0, n, k, tb), tb)
+    t = -(-n // 128) * -(-tb // 64)
+    assert rc == OK and names == ["mfma32_kernel"] and form() == ("0" if s == 1 else "1"), (n, k, tb, form())
+    assert fake.fake_blocks(fake.fake_launches() - 1) == (t if s == 1 else -(-t // 8) * 8 * s), (n, k, tb)
+""")
