@@ -38,27 +38,29 @@ __device__ __forceinline__ float block_max256(float v, float *red) {
 // reference's F32 router dot (moe.cpp:84-88), a serial double-precision sum in
 // k order.  Each product of two floats is exact in double, so every partial
 // sum rounds as the reference's does and the logit is its value bit for bit.
-// A workgroup owns one token and 64 experts.  The chain of dependent adds is
-// the bound, so nothing else is on it: waves 1..4 load 16 rows each, 256-byte
+// A workgroup owns one token and E experts.  The chain of dependent adds is
+// the bound, so nothing else is on it: waves 1..4 load E / 4 rows each, 256-byte
 // runs of a row per 16 lanes, three 64-value chunks ahead, and leave the
 // products in LDS ([value][expert], two chunks); wave 0, lane = expert, only
 // reads and adds.  Values past the row's end are products of 0 (a sum that
 // starts at +0 does not change by adding them).  16 tokens x 256 experts x
 // 2048 values: 27 us, about 30 clocks per dependent add; one thread per expert
-// with its loads on the chain took 280 us.
-constexpr int kRlC = 64;  // values per chunk
-template <bool VEC>       // 16-byte loads (n_embd % 4 == 0, gate_inp and x 16-byte aligned)
+// with its loads on the chain took 280 us.  E is 64, or 16 or 32 where that holds
+// every expert: with many tokens the products' LDS sets how many chains a CU
+// runs at once (8 experts, 2048 tokens: 86 us, 204 with E = 64).
+constexpr int kRlC = 64;       // values per chunk
+template <bool VEC, int E>     // VEC: 16-byte loads (n_embd % 4 == 0, gate_inp and x 16-byte aligned)
 __global__ __launch_bounds__(320) void route_logits_kernel(const float *__restrict__ x, int x_stride,
                                                            const float *__restrict__ gate_inp, int n_embd, int n_expert,
                                                            float *__restrict__ logits) {
-    __shared__ double prod[2][kRlC][65];
+    __shared__ double prod[2][kRlC][E + 1];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int e0 = blockIdx.x * 64, t = blockIdx.y;
+    const int e0 = blockIdx.x * E, t = blockIdx.y;
     const int nc = (n_embd + kRlC - 1) / kRlC;
-    const int kl = 4 * (lane & 15), rl = 16 * (wave - 1) + (lane >> 4);  // this lane's values and first row
+    const int kl = 4 * (lane & 15), rl = E / 4 * (wave - 1) + (lane >> 4);  // this lane's values and first row
     const float *xr = x + (size_t)t * x_stride;
     struct Piece {
-        float4 w[4], x;
+        float4 w[E / 16], x;
     } r[3];
     auto load4 = [&](const float *p, int k) {
         const int m = n_embd - 1;
@@ -69,7 +71,7 @@ __global__ __launch_bounds__(320) void route_logits_kernel(const float *__restri
         const int k = (c < nc ? c : nc - 1) * kRlC + kl;
         q.x = load4(xr, k);
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < E / 16; i++) {
             const int e = e0 + rl + 4 * i;
             q.w[i] = load4(gate_inp + (size_t)(e < n_expert ? e : n_expert - 1) * n_embd, k);
         }
@@ -80,7 +82,7 @@ __global__ __launch_bounds__(320) void route_logits_kernel(const float *__restri
 #pragma unroll
         for (int v = 0; v < 4; v++) in[v] = c * kRlC + kl + v < n_embd;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < E / 16; i++) {
             const float wv[4] = {q.w[i].x, q.w[i].y, q.w[i].z, q.w[i].w};
 #pragma unroll
             for (int v = 0; v < 4; v++)
@@ -109,22 +111,35 @@ __global__ __launch_bounds__(320) void route_logits_kernel(const float *__restri
     for (int c = 0; c < nc; c++) {
         __syncthreads();
         // sixteen reads ahead of the sixteen adds they feed
-        const double *p = &prod[c & 1][0][lane];
+        const double *p = &prod[c & 1][0][lane < E ? lane : 0];
         double v[2][16];
 #pragma unroll
-        for (int i = 0; i < 16; i++) v[0][i] = p[i * 65];
+        for (int i = 0; i < 16; i++) v[0][i] = p[i * (E + 1)];
 #pragma unroll
         for (int b = 0; b < kRlC / 16; b++) {
             if (b + 1 < kRlC / 16)
 #pragma unroll
-                for (int i = 0; i < 16; i++) v[(b + 1) & 1][i] = p[(16 * (b + 1) + i) * 65];
+                for (int i = 0; i < 16; i++) v[(b + 1) & 1][i] = p[(16 * (b + 1) + i) * (E + 1)];
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < 16; i++) a += v[b & 1][i];
             __builtin_amdgcn_sched_barrier(0);
         }
     }
-    if (e0 + lane < n_expert) logits[(size_t)t * n_expert + e0 + lane] = (float)a;
+    if (lane < E && e0 + lane < n_expert) logits[(size_t)t * n_expert + e0 + lane] = (float)a;
+}
+
+template <int E> static void route_logits(hipStream_t stream, const float *x, int x_stride, const float *gate_inp, int n_tok,
+                                          int n_embd, int n_expert, float *logits) {
+    for (int t0 = 0; t0 < n_tok; t0 += 65535) {  // tokens per launch: the grid's y limit
+        const dim3 grid((n_expert + E - 1) / E, n_tok - t0 < 65535 ? n_tok - t0 : 65535);
+        const float *xt = x + (size_t)t0 * x_stride;
+        float *lt = logits + (size_t)t0 * n_expert;
+        if (n_embd % 4 == 0 && x_stride % 4 == 0 && (uintptr_t)gate_inp % 16 == 0 && (uintptr_t)xt % 16 == 0)
+            hipLaunchKernelGGL((route_logits_kernel<true, E>), grid, dim3(320), 0, stream, xt, x_stride, gate_inp, n_embd, n_expert, lt);
+        else
+            hipLaunchKernelGGL((route_logits_kernel<false, E>), grid, dim3(320), 0, stream, xt, x_stride, gate_inp, n_embd, n_expert, lt);
+    }
 }
 
 __global__ __launch_bounds__(256) void route_kernel(int n_expert, int top_k, float *__restrict__ logits,
@@ -1243,15 +1258,9 @@ int miq_moe_route(hipStream_t stream, const float *x, int x_stride, const float 
     const int V = (n_expert + 63) / 64;
     const dim3 wgrid((n_tok + 3) / 4), wblock(256);
     if (gate_inp) {
-        for (int t0 = 0; t0 < n_tok; t0 += 65535) {  // tokens per launch: the grid's y limit
-            const dim3 grid(V, n_tok - t0 < 65535 ? n_tok - t0 : 65535);
-            const float *xt = x + (size_t)t0 * x_stride;
-            float *lt = logits + (size_t)t0 * n_expert;
-            if (n_embd % 4 == 0 && x_stride % 4 == 0 && (uintptr_t)gate_inp % 16 == 0 && (uintptr_t)xt % 16 == 0)
-                hipLaunchKernelGGL(miq::route_logits_kernel<true>, grid, dim3(320), 0, stream, xt, x_stride, gate_inp, n_embd, n_expert, lt);
-            else
-                hipLaunchKernelGGL(miq::route_logits_kernel<false>, grid, dim3(320), 0, stream, xt, x_stride, gate_inp, n_embd, n_expert, lt);
-        }
+        if (n_expert <= 16) miq::route_logits<16>(stream, x, x_stride, gate_inp, n_tok, n_embd, n_expert, logits);
+        else if (n_expert <= 32) miq::route_logits<32>(stream, x, x_stride, gate_inp, n_tok, n_embd, n_expert, logits);
+        else miq::route_logits<64>(stream, x, x_stride, gate_inp, n_tok, n_embd, n_expert, logits);
     }
     if (V <= 8) {  // up to 512 experts: one wave per token
         const int vv = V == 1 ? 1 : V == 2 ? 2 : V <= 4 ? 4 : 8;

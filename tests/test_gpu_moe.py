@@ -60,10 +60,10 @@ def test_route_gate_inp_near_ties(miq, oracle, dev):
 
 
 @pytest.mark.parametrize("n_tok,n_expert,n_embd,top_k", [
-    (1, 8, 1, 2), (3, 64, 63, 4), (2, 65, 64, 8), (5, 130, 65, 8), (2, 600, 196, 10), (4, 63, 2052, 6), (2, 256, 4098, 8)])
+    (1, 8, 1, 2), (3, 16, 260, 4), (2, 17, 129, 8), (3, 32, 64, 6), (2, 33, 128, 8), (3, 64, 63, 4), (2, 65, 64, 8), (5, 130, 65, 8), (2, 600, 196, 10), (4, 63, 2052, 6), (2, 256, 4098, 8)])
 @pytest.mark.parametrize("pad", [0, 1, 4])
 def test_route_gate_inp_sizes(miq, oracle, dev, n_tok, n_expert, n_embd, top_k, pad):
-    """Router logits around the kernel's 64-expert and 64-value tiles, with row strides
+    """Router logits around the kernel's 16-, 32- and 64-expert and 64-value tiles, with row strides
     and lengths that allow 16-byte loads and ones that do not: ids, weights and
     probabilities equal the oracle's serial double sum bit for bit."""
     import torch
