@@ -2,14 +2,15 @@
 //
 //   TB <= 3 (and the activation fits LDS)  dot4 GEMV (miq_gemv.hip)
 //   TB >= 33, Q4_K/Q5_K/Q6_K               exact fp16-MFMA GEMM, stream-K schedule (miq_pf16.hip),
-//                                          where its cost model beats the 16-token kernel;
-//                                          MIQ_PREFILL_FP16=0: the int8 kernel below
-//   TB >= 17, Q8_0 (and the switch above)  LDS-tiled 32x32 int8-MFMA GEMM (miq_mfma32.hip), where its
-//                                          cost model beats the 16-token kernel;
-//                                          Q6_K only when its tiles cover every CU
+//                                          where its cost model beats the 16-token kernel
+//   TB >= 17, Q8_0                         LDS-tiled 32x32 int8-MFMA GEMM (miq_mfma32.hip), where its
+//                                          cost model beats the 16-token kernel
 //   otherwise                              16-token int8-MFMA GEMM (miq_mfma16.hip)
-// The switch M32_MIN_TB (miq_set_switch, env MIQ_M32_MIN_TB; 17) moves the
-// smallest batch of both prefill kernels.
+// A/B switches (miq_set_switch, env MIQ_<name>).  PREFILL_FP16=2: every K-quant
+// batch from 48 tokens on is the fp16 GEMM's; 0: every batch from 48 tokens on
+// the int8 tiled GEMM's (Q6_K only when its tiles cover every CU).
+// M32_MIN_TB=n: the prefill kernels from n tokens on instead of 17 / 33 / 48
+// (0, the default).
 #include "miq_internal.h"
 
 namespace miq {
@@ -19,7 +20,6 @@ enum Route { kRouteGemv, kRoutePf16, kRouteM32, kRouteM16, kRouteQ80, kRouteNone
 
 Route route(const miq_seg *s, int TB) {
     if (q80_any(s)) return kRouteQ80;  // Q8_0 with an odd group count: its own kernel at every batch size
-    const int min_tb32 = sw(kSwM32MinTb);
     // GEMV_MAX_TB: the largest batch the dot4 GEMV takes (an A/B switch)
     const int gemv_max = sw(kSwGemvMaxTb);
     if (TB <= gemv_max && gemv_fits(s, TB)) return kRouteGemv;
@@ -29,10 +29,13 @@ Route route(const miq_seg *s, int TB) {
     const int pf_mode = sw(kSwPrefillFp16);
     // Inside miq_i8_gemm_noalloc every batch below 48 tokens is the 16-token
     // kernel's and every larger Q8_0 one the int8 GEMM's, whatever the models say.
+    // Below 48 tokens the models are what makes the prefill kernels the faster
+    // ones: with PREFILL_FP16=0, which asks none, 17 tokens of 7168 x 5120 Q4_K
+    // take 28 us against the 16-token kernel's 15.
     const bool fixed = static_scratch_mode();
-    const int min_tb = fixed && min_tb32 < 48 ? 48 : min_tb32;
+    const int set_tb = sw(kSwM32MinTb), min_tb = set_tb ? set_tb : fixed || pf_mode != 1 ? 48 : 17;
     const bool pf16 = pf_mode == 2 || (pf_mode == 1 && pf16_serves(s) &&
-                                       (fixed ? pf16_refuses_noalloc(s, TB) : TB > 32 && pf16_prefers(s, TB)));
+                                       (fixed ? pf16_refuses_noalloc(s, TB) : (set_tb || TB > 32) && pf16_prefers(s, TB)));
     if (TB >= min_tb && pf16 && pf16_serves(s)) return kRoutePf16;
     if (TB >= min_tb && (pf_mode == 0 || !pf16_serves(s)) && mfma32_serves(s) && mfma32_fills(s, TB) &&
         (pf_mode == 0 || fixed || mfma32_prefers(s, TB)))
@@ -42,19 +45,22 @@ Route route(const miq_seg *s, int TB) {
 }
 
 // The int8 tiled GEMM needs no scratch to run (unsliced), so its batches may
-// overlap on several streams of a device: from 48 tokens on, whichever kernel
-// then takes them, their partials are in scratch of the stream's own or there
-// are none.  Below that they share the device's scratch as the 16-token
-// kernel's batches do.
+// overlap on several streams of a device: from 48 tokens on (where it is set,
+// from M32_MIN_TB on), whichever kernel then takes them, their partials are in
+// scratch of the stream's own or there are none.  Below that they share the
+// device's scratch as the 16-token kernel's batches do.
 bool own_scratch(const miq_seg *s, int TB) {
-    return TB >= 48 && !q80_any(s) && mfma32_serves(s) && (s->type == MIQ_TYPE_Q8_0 || route(s, TB) == kRouteM32);
+    const int set_tb = sw(kSwM32MinTb);
+    return TB >= (set_tb ? set_tb : 48) && !q80_any(s) && mfma32_serves(s) &&
+           (s->type == MIQ_TYPE_Q8_0 || route(s, TB) == kRouteM32);
 }
 }  // namespace
 
 int run_gemm(hipStream_t stream, const miq_seg *s, int TB, const char *who) {
     const int rc = check_seg(s, TB, who);
     if (rc != MIQ_OK) return rc;
-    const OwnScratch scope(own_scratch(s, TB));
+    const bool own = own_scratch(s, TB);
+    const OwnScratch scope(own);
     switch (route(s, TB)) {
     case kRouteGemv: return launch_gemv(stream, s, TB);
     case kRoutePf16: {
@@ -69,7 +75,7 @@ int run_gemm(hipStream_t stream, const miq_seg *s, int TB, const char *who) {
     case kRouteM16: {
         const int rc = launch_mfma16(stream, s, TB);
         // no scratch (the stream captures a graph, or has none of its own): Q8_0 prefill batches still run, unsliced
-        if (rc == MIQ_UNSUPPORTED && s->type == MIQ_TYPE_Q8_0 && TB >= sw(kSwM32MinTb) && mfma32_serves(s))
+        if (rc == MIQ_UNSUPPORTED && own)
             return launch_mfma32(stream, s, TB);
         return rc;
     }

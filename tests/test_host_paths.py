@@ -197,3 +197,37 @@ for n, k, tb, s in ((17408, 5120, 333, 1), (5120, 5120, 512, 1), (5120, 512, 100
     assert rc == OK and names == ["mfma32_kernel"] and form() == ("0" if s == 1 else "1"), (n, k, tb, form())
     assert fake.fake_blocks(fake.fake_launches() - 1) == (t if s == 1 else -(-t // 8) * 8 * s), (n, k, tb)
 """)
+
+
+ROUTES = r"""
+def kernel(qt, n, k, tb, fn="i8_gemm"):
+    rc, names, _ = run(fn, seg(qt, n, k, tb), tb)
+    assert rc == OK, rc
+    return names[-1]
+want = %r
+for (qt, tb), k in want.items():
+    assert kernel(qt, 17408, 5120, tb) == k + "_kernel", (qt, tb, kernel(qt, 17408, 5120, tb))
+"""
+
+
+@pytest.mark.parametrize("env,want", [
+    ({}, {(12, 32): "m16z", (12, 33): "pf16", (8, 16): "m16z", (8, 17): "mfma32", (14, 48): "pf16"}),
+    # the forced forms from 48 tokens on: below, no model says that they are the faster ones
+    ({"MIQ_PREFILL_FP16": "0"}, {(12, 47): "m16z", (12, 48): "mfma32", (8, 47): "m16z", (8, 48): "mfma32", (14, 17): "m16z"}),
+    ({"MIQ_PREFILL_FP16": "2"}, {(12, 47): "m16z", (12, 48): "pf16", (14, 47): "m16z", (14, 48): "pf16"}),
+    ({"MIQ_PREFILL_FP16": "2", "MIQ_M32_MIN_TB": "17"}, {(12, 16): "m16z", (12, 17): "pf16"}),
+    ({"MIQ_PREFILL_FP16": "0", "MIQ_M32_MIN_TB": "20"}, {(12, 19): "m16z", (12, 20): "mfma32"}),
+    ({"MIQ_M32_MIN_TB": "100"}, {(12, 99): "m16z", (12, 100): "pf16", (8, 99): "m16z"}),
+])
+def test_smallest_prefill_batches(host, env, want):
+    """the smallest batches of the prefill kernels by default and under the switches that force one"""
+    host(ROUTES % want, **env)
+
+
+def test_noalloc_smallest_prefill_batches(host):
+    """miq_i8_gemm_noalloc keeps the 16-token kernel below 48 tokens, whatever miq_i8_gemm does there"""
+    host(r"""
+for qt, tb, want in ((Q4_K, 40, "m16z_kernel"), (Q8_0, 20, "m16z_kernel"), (Q8_0, 47, "m16z_kernel"), (Q8_0, 48, "mfma32_kernel")):
+    rc, names, _ = run("i8_gemm_noalloc", seg(qt, 7168, 5120, tb), tb)
+    assert rc == OK and names == [want], (qt, tb, rc, names)
+""")
