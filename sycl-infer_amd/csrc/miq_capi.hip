@@ -301,7 +301,8 @@ struct SwitchDef {
 // names (the environment variable is MIQ_<name>) and defaults, in Switch order
 constexpr SwitchDef kSwitches[kSwCount] = {
     {"M32_MIN_TB", 0}, {"GEMV_MAX_TB", 3}, {"PREFILL_FP16", 1}, {"FUSED_QUANT", 1},
-    {"M16_WAVES", 0},   {"M16_FORM", 0},    {"MOE_GRP", 1},      {"M32_FILL", 1}};
+    {"M16_WAVES", 0},   {"M16_FORM", 0},    {"MOE_GRP", 1},      {"M32_FILL", 1},
+    {"XCD_ASTRAY", 0}};
 std::atomic<int> g_sw[kSwCount];
 std::once_flag g_sw_once;
 

@@ -28,7 +28,7 @@ bool static_scratch_mode();
 // environment variable MIQ_<name>, read once per process, else its default;
 // miq_set_switch() changes it at run time.
 enum Switch {
-    kSwM32MinTb, kSwGemvMaxTb, kSwPrefillFp16, kSwFusedQuant, kSwM16Waves, kSwM16Form, kSwMoeGrp, kSwM32Fill, kSwCount
+    kSwM32MinTb, kSwGemvMaxTb, kSwPrefillFp16, kSwFusedQuant, kSwM16Waves, kSwM16Form, kSwMoeGrp, kSwM32Fill, kSwXcdAstray, kSwCount
 };
 int sw(Switch s);
 // Compute units of the current device (queried once per device).

@@ -166,8 +166,12 @@ __device__ __forceinline__ void wload(typename WOf<TYPE>::T &W, __amdgpu_buffer_
 // the S partials in slice order -- deterministic whatever the arrival order --
 // applies alpha and the residual and re-arms the counter.  The partials meet
 // in the XCD's L2 (stores drained before the arrival is counted, L1-bypassing
-// loads); a workgroup that finds itself on another XCD (HW_REG_XCC_ID) falls
-// back to agent-scope fences and marks the counter so the reducer fences too.
+// loads).  A workgroup that finds itself on another XCD (HW_REG_XCC_ID) uses
+// agent-scope fences and marks the counter so the reducer fences too.  That
+// covers a launch whose workgroups are all shifted to other XCDs, and a
+// misplaced slice that a well-placed one reduces; it does not cover a misplaced
+// last slice of a tile whose others are in place (they wrote nothing back past
+// their L2).  The dispatcher's round-robin placement produces neither.
 constexpr size_t kZSlotX = 8 * 512;    // codes of one K step: [group][h][token][8 B]
 constexpr size_t kZSlotM = 8 * 16 * 4; // one fp32 per (group, token)
 constexpr int kZXcd = 8;
@@ -759,7 +763,7 @@ __global__ __launch_bounds__(64 * kCWaves, 1) void m16c_kernel(CArgs P) {
         }
         constexpr uint32_t kFar = 1u << 20;
         *reinterpret_cast<v4f *>(P.part + ((size_t)tile * P.KP + kp) * 256 + lane * 4) = val;
-        if (far) __threadfence();  // the part's partner may sit on another XCD
+        if (far) __threadfence();  // misplaced: see the split-K form above for what this covers
         __builtin_amdgcn_s_waitcnt(0);
         uint32_t prev = 0;
         if (lane == 0) prev = __hip_atomic_fetch_add(P.cnt + tile, far ? 1u + kFar : 1u, __ATOMIC_RELAXED,

@@ -52,6 +52,7 @@ struct M32Args {
     int S;          // K slices per tile
     float *part;    // [tile][slice][8][256 threads][4] partial sums (S > 1)
     uint32_t *cnt;  // [tile] arrival counters, zero between launches
+    int astray;     // a test: every second slice takes itself for one on another XCD
 };
 
 // LDS layout of one step
@@ -255,17 +256,20 @@ __global__ __launch_bounds__(256, 2) void mfma32_kernel(M32Args A) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wt = (wave >> 1) * 32, wn = (wave & 1) * 64;  // wave tile origin (tokens, rows)
     const int l32 = lane & 31, hk = lane >> 5;
-    int kb0 = 0, nkb = A.K / 256;
-    if constexpr (FORM == kM32Sliced) {
-        kb0 = slice * (A.K / 256) / A.S;
-        nkb = (slice + 1) * (A.K / 256) / A.S;
-    }
     const __amdgpu_buffer_rsrc_t rw = make_rsrc(A.w, A.w_bytes);
     const uint32_t xbytes = (uint32_t)(A.K / 32) * A.TB * 32, mbytes = (uint32_t)(A.K / 32) * A.TB * 8;
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(A.x8, xbytes);
     const __amdgpu_buffer_rsrc_t rm = make_rsrc(A.xmeta, mbytes), rq = make_rsrc(A.xsumq, mbytes);
 
-    v16f acc[2], t2[2];
+    v16f acc[2];
+    const int steps = A.K / 256;
+    int kb0 = 0, nkb = steps;  // this workgroup's steps of the tile
+    if constexpr (FORM == kM32Sliced) {
+        kb0 = slice * steps / A.S;
+        nkb = (slice + 1) * steps / A.S;
+    }
+    v16f t2[2];
+sum_steps:
 #pragma unroll
     for (int j = 0; j < 2; j++) {
         acc[j] = v16f{};
@@ -380,21 +384,25 @@ __global__ __launch_bounds__(256, 2) void mfma32_kernel(M32Args A) {
             }
         }
     }
-    if constexpr (DOTS) return;
 #pragma unroll
     for (int j = 0; j < 2; j++) acc[j] -= t2[j];
-    if constexpr (FORM == kM32Sliced) {
+    if constexpr (DOTS) return;
+    if (FORM == kM32Sliced && nkb - kb0 < steps) {
         // The last slice of a tile to arrive adds the slices in slice order (the
         // result does not depend on timing); one that finds every other one
         // arrived keeps its sums in registers.  The partials meet in the XCD's
         // L2 (stores drained before the arrival is counted, L1-bypassing
-        // loads); a workgroup on another XCD than expected (HW_REG_XCC_ID)
-        // fences and marks the counter so that the reducer fences too.
+        // loads).  A workgroup on another XCD than expected (HW_REG_XCC_ID; the
+        // dispatcher places none there) writes its partial back past its L2 and
+        // marks the counter so that the reducer drops stale lines first; where
+        // it is itself the last, it cannot see the others' partials and computes
+        // the whole tile instead, in one sum.
         __shared__ int lflag;
         constexpr uint32_t kFar = 1u << 20;
         v4f32 *P = reinterpret_cast<v4f32 *>(A.part) + (size_t)tile * A.S * 2048 + threadIdx.x;
         uint32_t *cnt = A.cnt + tile;
-        const bool far = (__builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 15) != (uint32_t)(blockIdx.x & 7);
+        const bool far = (__builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 15) != (uint32_t)(blockIdx.x & 7) ||
+                         (A.astray && (slice & 1));
         if (threadIdx.x == 0) {
             const uint32_t prev = __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             lflag = (prev & (kFar - 1)) == (uint32_t)(A.S - 1) ? 1 + (prev >= kFar) : 0;
@@ -421,7 +429,12 @@ __global__ __launch_bounds__(256, 2) void mfma32_kernel(M32Args A) {
             fl = __builtin_amdgcn_readfirstlane(lflag);
         }
         if (!fl) return;
-        if (fl == 2 || far) __threadfence();
+        if (far) {
+            kb0 = 0;
+            nkb = steps;
+            goto sum_steps;
+        }
+        if (fl == 2) __threadfence();
         v16f sum[2] = {};
         const __amdgpu_buffer_rsrc_t rp = make_rsrc(reinterpret_cast<v4f32 *>(A.part) + (size_t)tile * A.S * 2048, (uint32_t)A.S * 32768u);
         for (int k = 0; k < A.S; k++) {
@@ -529,6 +542,7 @@ int launch_mfma32(hipStream_t stream, const miq_seg *s, int TB, int32_t *dots) {
     // no scratch for the partials (a stream that captures a graph or has none of
     // its own, miq_i8_gemm_noalloc): unsliced
     if (A.S > 1 && scratch_get(stream, (size_t)A.T * A.S * 32768, A.T, &A.part, &A.cnt) != MIQ_OK) A.S = 1;
+    A.astray = sw(kSwXcdAstray);
     const M32Form form = dots ? kM32Dots : A.S > 1 ? kM32Sliced : kM32Whole;
     const dim3 grid((unsigned)(form == kM32Sliced ? (A.T + 7) / 8 * 8 * A.S : A.T));
     A.dots = dots;  // the parity form is miq_group_dots path 3

@@ -103,6 +103,7 @@ struct PfArgs {
     float *part;   // per matrix [2 * workgroups] slots of [2*TT][512 threads][4] partial sums (stream-K)
     uint32_t *cnt; // per matrix [tile] arrival counters, zero between launches
     int32_t *dots; // parity form: [TB][n_rows][K/32] MFMA group results
+    int astray;    // a test: every second workgroup of an XCD takes itself for one on another
     PfSeg seg[kPfSegs];
 };
 
@@ -751,9 +752,12 @@ __global__ __launch_bounds__(kPT, 2) void pf16_kernel(PfArgs A) {
     // range is stored directly; otherwise each range writes a partial (slot 2v
     // for the tile it starts in, 2v+1 for the one it ends in), and the last
     // contributor to arrive adds the partials in range order (the result does
-    // not depend on timing) and stores.  The partials of a tile stay in their
-    // XCD's L2 unless a workgroup finds itself on another XCD than
-    // blockIdx % 8, or G == 1: then they go through memory.
+    // not depend on timing) and stores.  With G == 1 the partials go through
+    // memory, else those of a tile stay in their XCD's L2.  A workgroup that finds
+    // itself on another XCD than blockIdx % 8 (the dispatcher places none there)
+    // writes its partial back past its L2 and marks the counter so that the
+    // reducer drops stale lines first; where it is itself the last to arrive, it
+    // cannot see the others' partials and computes the whole tile, in one sum.
     constexpr uint32_t kFar = 1u << 20;
     constexpr int kPart = 2 * TT * kPT;  // f4 of one partial tile
     const int w = blockIdx.x;
@@ -762,7 +766,7 @@ __global__ __launch_bounds__(kPT, 2) void pf16_kernel(PfArgs A) {
     const int P = S.P;
     if (w >= P) continue;
     const int T = S.nt * A.mt;
-    const int F = S.rounds * P, sk = T - F;
+    const int F = S.rounds * P, sk = T > F ? T - F : 0;  // no stream-K tiles where the last round is not full (DOTS)
     const bool xmap = S.xmap;
     const int G = xmap ? 8 : 1, x = xmap ? w % 8 : 0, Pg = P / G, vl = xmap ? w / 8 : w;
     f4 *part = reinterpret_cast<f4 *>(A.part) + (size_t)S.poff * kPart;
@@ -775,6 +779,9 @@ __global__ __launch_bounds__(kPT, 2) void pf16_kernel(PfArgs A) {
     auto owner = [&](int blk) { return blk < rr * (rq + 1) ? blk / (rq + 1) : rr + (blk - rr * (rq + 1)) / rq; };
     const int bs = rstart(vl), be = rstart(vl + 1);
     const int v = x * Pg + vl;  // global range id (partial slots)
+    // Added to b0 (at most 2^30 blocks): compute the last piece's tile again.  A
+    // variable of its own cost up to 1.5 % of the launch.
+    constexpr int kAgain = 1 << 30;
     int k = 0, b0 = bs;
     for (;;) {
         // next segment: a data-parallel tile, else the next piece of this
@@ -794,12 +801,18 @@ __global__ __launch_bounds__(kPT, 2) void pf16_kernel(PfArgs A) {
             t = tx0 + lt;
             kb0 = b0 - lt * nkb;
             kb1 = be - lt * nkb < nkb ? be - lt * nkb : nkb;
+        } else if (__builtin_expect(b0 >= kAgain, 0)) {
+            dp = true;
+            b0 -= kAgain;
+            t = tx0 + (b0 - 1) / nkb;
+            kb0 = 0;
+            kb1 = nkb;
         } else {
             break;
         }
         const int n0 = t / A.mt * kPN, tg = t % A.mt;
         run(S, n0, tg, kb0, kb1);
-        if (dp) {  // a data-parallel tile
+        if (dp) {  // a whole tile
             if constexpr (!DOTS) store(S, n0, tg);
             continue;
         }
@@ -813,7 +826,9 @@ __global__ __launch_bounds__(kPT, 2) void pf16_kernel(PfArgs A) {
         const int v_lo = owner(tb0), v_hi = owner(tb1 - 1);
         int n_contrib = 0;  // ranges of the tile that hold a block (with few blocks some are empty)
         for (int u = v_lo; u <= v_hi; u++) n_contrib += rstart(u) < rstart(u + 1);
-        const bool far = !xmap || (__builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 15) != (uint32_t)x;  // HW_REG_XCC_ID
+        const bool astray = xmap && ((__builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 15) != (uint32_t)x ||  // HW_REG_XCC_ID
+                                     (A.astray && (vl & 1)));
+        const bool far = !xmap || astray;
         // A range that finds every other one arrived keeps its sums in registers.
         if (tid == 0) {
             const uint32_t prev = __hip_atomic_load(cnt + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -844,6 +859,10 @@ __global__ __launch_bounds__(kPT, 2) void pf16_kernel(PfArgs A) {
             fl = __builtin_amdgcn_readfirstlane(lflag);
         }
         if (!fl) continue;
+        if (__builtin_expect(astray, 0)) {
+            b0 += kAgain;
+            continue;
+        }
         if (fl == 2 || far) __threadfence();  // some partial crossed XCDs: drop stale L2 lines first
         f4 sum[2][TT];
 #pragma unroll
@@ -1000,6 +1019,7 @@ static int launch(hipStream_t stream, const miq_seg *segs, int n_segs, int TB, i
     A.K = K;
     A.TB = TB;
     A.dots = dots;
+    A.astray = sw(kSwXcdAstray);
     int n_cu = 0;
     if (const int rc = device_cus(&n_cu)) return rc;
     if (const int rc = pf_lds_limit()) return rc;

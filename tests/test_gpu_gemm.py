@@ -492,6 +492,45 @@ def test_gemm_prefill_int8_slices(miq, oracle, dev, qt, TB, N, K, switch):
     assert_elem(got[:TB, :N], exp, elem_bound(oracle, qt, wq, K, a, 0.5), residual=res[:, :N])
 
 
+@pytest.mark.parametrize("qt,TB,N,K", [(Q8_0, 130, 1100, 5376), (Q8_0, 333, 5120, 4096), (Q4_K, 130, 2100, 2304), (Q5_K, 77, 4400, 5120),
+                                       (Q6_K, 256, 3000, 1024)])
+def test_prefill_partials_across_xcds(miq, oracle, dev, qt, TB, N, K, switch):
+    """Both prefill GEMMs where every second workgroup that shares a tile takes itself
+    for one on another XCD (XCD_ASTRAY): its partial goes through memory, and where it
+    is the last it computes the tile again.  Within the per-output bound in every run,
+    with the normal placement's bits back afterwards."""
+    import torch
+    print(f"prefill across XCDs qt={qt} TB={TB} N={N} K={K}", flush=True)
+    switch("PREFILL_FP16", "2")
+    wq = weights(miq, qt, N, K, seed=TB + N)
+    rng = np.random.default_rng(TB + K)
+    x = rng.standard_normal((TB, K)).astype(np.float32)
+    res = rng.standard_normal((TB, N)).astype(np.float32)
+    act = miq.xq(to_dev(x, dev))
+    wd, rd = to_dev(wq, dev), to_dev(res, dev)
+
+    def run():
+        out = torch.full((TB, N), float("nan"), dtype=torch.float32, device=dev)
+        miq.i8_gemm(miq.make_seg(wd, qt, K, N, act, out, N, residual=rd, alpha=0.5), TB)
+        torch.cuda.synchronize()
+        return out.cpu().numpy()
+
+    normal = run()
+    a = oracle.xq(x)
+    exp = 0.5 * oracle.gemm(qt, wq, K, N, a) + res
+    bound = elem_bound(oracle, qt, wq, K, a, 0.5)
+    assert_elem(normal, exp, bound, residual=res)
+    switch("XCD_ASTRAY", "1")
+    differ = 0
+    for _ in range(8):
+        got = run()
+        assert_elem(got, exp, bound, residual=res)
+        differ += int((got != normal).sum())
+    assert differ  # some tile was computed in one sum
+    switch("XCD_ASTRAY", "0")
+    assert np.array_equal(run().view(np.uint32), normal.view(np.uint32))
+
+
 @pytest.mark.parametrize("TB,N,K", [(200, 5120, 2560), (64, 1024, 5120)])
 def test_q80_prefill_streams_overlap(miq, oracle, dev, TB, N, K):
     """Q8_0 prefill (K slices; a small matrix on the 16-token kernel) queued on two
