@@ -1,9 +1,10 @@
 """GPU parity across the batch-size dispatch: every type at token counts on both
 sides of each cut-off the library routes by -- the GEMV (1..3 tokens), the
-16-token int8-MFMA GEMM (4..47), the prefill GEMMs (48 and up, where the
-cost model picks between the fp16 GEMM and the 16-token kernel) -- on a shape
-whose rows leave partial tiles everywhere (N = 260) and K = 2304 (nine blocks:
-odd slice counts).  Each output is checked against the oracle (the normwise
+16-token int8-MFMA GEMM, the prefill GEMMs (Q8_0 from 17 tokens, the others
+from 33, where their cost models beat the 16-token kernel; for a matrix as small
+as this that is Q8_0 only, the fp16 GEMM's own sizes are in test_gpu_gemm.py) --
+on a shape whose rows leave partial tiles everywhere (N = 260) and K = 2304 (nine
+blocks: odd slice counts).  Each output is checked against the oracle (the normwise
 1e-4 bound and the per-output summation-order bound), and the fused entry point
 (miq_quant_gemm) must equal miq_xq + miq_i8_gemm bit for bit."""
 import numpy as np

@@ -330,7 +330,7 @@ def test_gemm_prefill_q6k_vs_oracle(miq, oracle, dev, TB, N, K, form, switch):
                                     (384, 21888, 512), (256, 4352, 2304)])
 def test_gemm_prefill_fp16_vs_oracle(miq, oracle, dev, qt, TB, N, K, switch):
     """The exact fp16-MFMA prefill GEMM (q*sc against x8, sx per group in fp32,
-    128 x 128 tiles; the dmin term on bf16 MFMA with a three-term split):
+    256 rows x up to 128 tokens; the dmin term on bf16 MFMA with a three-term split):
     partial row / token tiles, residual and alpha.  Small shapes run as K-split
     parts of a few tiles (stream-K)."""
     print(f"prefill qt={qt} TB={TB} N={N} K={K}", flush=True)
@@ -412,14 +412,16 @@ def test_gemm_cu_form_default_many_tiles(miq, oracle, dev):
 
 
 @pytest.mark.parametrize("qt", [Q4_K, Q5_K, Q6_K])
-@pytest.mark.parametrize("TB,N,K", [(48, 1, 256), (64, 255, 256), (65, 256, 512), (96, 257, 768), (97, 31, 2304), (128, 600, 512),
+@pytest.mark.parametrize("TB,N,K", [(17, 300, 512), (31, 256, 768), (32, 257, 2304), (48, 1, 256), (64, 255, 256), (65, 256, 512), (96, 257, 768), (97, 31, 2304), (128, 600, 512),
                                     (129, 33, 256), (160, 512, 1024), (257, 300, 768)])
 def test_gemm_prefill_tile_edges(miq, oracle, dev, qt, TB, N, K, switch):
-    """The fp16 GEMM at the edges of its tiles (256 rows of 32-row waves; 32, 64, 96 and
-    128 tokens), of one K block per range and of uneven ranges, with a strided output and
-    a residual: the per-output summation-order bound, nothing written beside the outputs."""
+    """The fp16 GEMM at the edges of its tiles (256 rows of 32-row waves; token tiles of
+    two to eight sixteens), of one K block per range and of uneven ranges, with a strided
+    output and a residual: the per-output summation-order bound, nothing written beside
+    the outputs."""
     import torch
     switch("PREFILL_FP16", "2")
+    switch("M32_MIN_TB", "17")
     wq = weights(miq, qt, N, K, seed=TB * 7 + N)
     rng = np.random.default_rng(TB + K)
     x = rng.standard_normal((TB, K)).astype(np.float32)
@@ -572,6 +574,39 @@ def test_q80_prefill_streams_overlap(miq, oracle, dev, TB, N, K):
     assert_elem(go.cpu().numpy(), oracle.gemm(Q8_0, wqs[0], K, N, a), elem_bound(oracle, Q8_0, wqs[0], K, a, 1.0))
 
 
+@pytest.mark.parametrize("qt", [Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("up", [False, True])
+@pytest.mark.parametrize("TB,N,K", [(17, 40, 256), (33, 300, 768), (77, 260, 2304), (130, 33, 512), (512, 500, 256)])
+def test_quant_gemm_prefill_pre_pass(miq, oracle, dev, qt, up, TB, N, K, switch):
+    """miq_quant_gemm on the fp16 GEMM, whose pre-pass quantizes: x8, xmeta and xsumq
+    equal miq_xq's byte for byte and the output miq_xq + miq_i8_gemm's bit for bit, with
+    and without silu(x) * up, from activations with a row stride above K, groups of
+    zeros, ties and a wide range; the output within its bound of the oracle."""
+    import torch
+    print(f"quant gemm prefill pre-pass qt={qt} up={up} TB={TB} N={N} K={K}", flush=True)
+    switch("PREFILL_FP16", "2")
+    switch("M32_MIN_TB", "17")
+    wq = weights(miq, qt, N, K, seed=TB + qt)
+    rng = np.random.default_rng(TB + K)
+    xp, upad = (rng.standard_normal((TB, K + 12)).astype(np.float32) * 3 for _ in range(2))
+    xp[:, 32:64] = 0
+    xp[0, 64:96] = np.round(xp[0, 64:96] * 2) / 2  # ties of the rounding
+    xp[TB // 2] *= 1e-5
+    x, u = to_dev(xp, dev)[:, :K], to_dev(upad, dev)[:, :K] if up else None
+    wd = to_dev(wq, dev)
+    ref_act, act = miq.alloc_act(TB, K, dev), miq.alloc_act(TB, K, dev)
+    ref, out = (torch.full((TB, N), float("nan"), dtype=torch.float32, device=dev) for _ in range(2))
+    miq.xq(x, u, out=ref_act)
+    miq.i8_gemm(miq.make_seg(wd, qt, K, N, ref_act, ref, N), TB)
+    miq.quant_gemm(miq.make_seg(wd, qt, K, N, act, out, N, x=x, act_up=u), TB)
+    torch.cuda.synchronize()
+    for name in ("x8", "xmeta", "xsumq"):
+        assert torch.equal(getattr(act, name).view(torch.int8).cpu(), getattr(ref_act, name).view(torch.int8).cpu()), name
+    assert torch.equal(out.cpu().view(torch.int32), ref.cpu().view(torch.int32))
+    a = oracle.xq(np.ascontiguousarray(xp[:, :K]), np.ascontiguousarray(upad[:, :K]) if up else None)
+    assert_elem(out.cpu().numpy(), oracle.gemm(qt, wq, K, N, a), elem_bound(oracle, qt, wq, K, a, 1.0))
+
+
 @pytest.mark.parametrize("TB,K,rows", [(77, 512, (300, 256, 17)), (200, 768, (1024, 40)), (512, 256, (2048, 4352)),
                                        (512, 2304, (2048,) * 6)])
 def test_quant_gemm_multi_prefill(miq, dev, TB, K, rows, switch):
@@ -596,7 +631,7 @@ def test_quant_gemm_multi_prefill(miq, dev, TB, K, rows, switch):
 
 
 def test_gemm_prefill_fp16_stream_k(miq, oracle, dev, switch):
-    """512 x 16640: 520 tiles of 128 x 128 on 512 resident workgroups, so every
+    """512 x 16640: 260 tiles of 256 rows x 128 tokens on 256 workgroups, so every
     tile's K blocks are dealt out as contiguous ranges (stream-K), partial sums
     met in the XCD's L2 and added in range order."""
     print("prefill stream-K", flush=True)
@@ -672,13 +707,14 @@ def test_fused_quant_gemm_equals_two_calls(miq, dev):
 
 @pytest.mark.parametrize("N,K,TB,up", [(17408, 5120, 16, False), (5120, 17408, 16, False), (17408, 5120, 8, True),
                                         (17408, 5120, 33, False), (2048, 5120, 5, False), (4096, 5120, 33, True)])
-def test_quant_gemm_sixteen_token_routes(miq, oracle, dev, N, K, TB, up):
+def test_quant_gemm_sixteen_token_routes(miq, oracle, dev, N, K, TB, up, switch):
     """miq_quant_gemm on the 16-token routes (the bounded split-K form for the first
     four shapes, the all-at-entry form for the last two): the output equals miq_xq +
     miq_i8_gemm bit for bit and x8 / xmeta / xsumq equal miq_xq's, over three calls
     in a row on the same buffers."""
     import torch
     print(f"quant gemm 16-token route N={N} K={K} TB={TB} up={up}", flush=True)
+    switch("M32_MIN_TB", "48")  # 33 tokens of the largest matrix are the fp16 GEMM's by default
     wq = weights(miq, Q4_K, N, K, seed=N + K + TB)
     rng = np.random.default_rng(TB + K)
     x = to_dev(rng.standard_normal((TB, K)).astype(np.float32), dev)

@@ -48,9 +48,29 @@ def _segs(miq, dev, specs, K, TB, seed):
     ([(Q4_K, 500, False, 1.0), (Q5_K, 300, True, 1.0)], 2048, 16),      # mixed types: one launch each
     ([(Q4_K, 640, False, 1.0), (Q4_K, 129, True, 1.0)], 1024, 4),       # the split-K kernel's smallest batch
     ([(Q6_K, 333, False, 1.0), (Q6_K, 1024, False, 1.0)], 2048, 47),    # its largest (three token tiles)
-    ([(Q4_K, 2048, False, 1.0), (Q4_K, 512, False, 1.0)], 2048, 64),    # prefill sizes: one GEMM per segment
+    ([(Q4_K, 2048, False, 1.0), (Q4_K, 512, False, 1.0)], 2048, 64),    # small matrices: the split-K launch
 ])
 def test_multi_matches_single(miq, oracle, dev, specs, K, TB, fused):
+    _multi_matches_single(miq, oracle, dev, specs, K, TB, fused)
+
+
+@pytest.mark.parametrize("fused", [True, False])
+@pytest.mark.parametrize("pf,specs,K,TB", [
+    # one launch of the fp16 prefill GEMM over every segment: forced, and by the default rule
+    ("2", [(Q4_K, 700, True, 0.5), (Q4_K, 2100, False, 1.0), (Q4_K, 33, True, 1.0)], 1024, 64),
+    ("2", [(Q5_K, 300, True, 2.0), (Q5_K, 1000, True, 1.0)], 2304, 130),
+    ("2", [(Q6_K, 257, False, 1.0), (Q6_K, 64, True, 0.25)], 512, 48),
+    ("1", [(Q6_K, 7168, True, 1.0), (Q6_K, 7168, False, 1.0)], 5120, 96),
+    # Q8_0 and mixed types: one launch each
+    ("1", [(Q8_0, 2048, True, 1.0), (Q8_0, 1000, False, 0.5)], 4096, 100),
+    ("2", [(Q4_K, 300, True, 1.0), (Q6_K, 500, True, 1.0)], 768, 77),
+])
+def test_multi_prefill_matches_single(miq, oracle, dev, specs, K, TB, fused, pf, switch):
+    switch("PREFILL_FP16", pf)
+    _multi_matches_single(miq, oracle, dev, specs, K, TB, fused)
+
+
+def _multi_matches_single(miq, oracle, dev, specs, K, TB, fused):
     import torch
     print(f"multi fused={fused} K={K} TB={TB} segs={[(s[0], s[1]) for s in specs]}", flush=True)
     x, act, segs = _segs(miq, dev, specs, K, TB, seed=K + TB + len(specs))

@@ -231,3 +231,28 @@ for qt, tb, want in ((Q4_K, 40, "m16z_kernel"), (Q8_0, 20, "m16z_kernel"), (Q8_0
     rc, names, _ = run("i8_gemm_noalloc", seg(qt, 7168, 5120, tb), tb)
     assert rc == OK and names == [want], (qt, tb, rc, names)
 """)
+
+
+def test_capture_without_workspace(host):
+    """a capturing stream and a prefill shape that was not run before: the 16-token kernel where it has its scratch
+    and miq_i8_gemm_noalloc would use it too, else a refusal before anything runs; Q8_0 runs unsliced"""
+    host(r"""
+fake.fake_capturing(1)
+small, large = seg(Q4_K, 17408, 5120, 40), seg(Q4_K, 17408, 5120, 512)
+for fn in ("i8_gemm", "i8_gemv_multi"):
+    assert run(fn, small, 40)[:2] == (UNSUPPORTED, []) and run(fn, large, 512)[:2] == (UNSUPPORTED, [])
+rc, names, bufs = run("i8_gemm", seg(Q8_0, 5120, 5120, 40), 40)
+assert rc == OK and names == ["mfma32_kernel"] and not bufs[0] and not sliced(5120, 40)
+fake.fake_capturing(0)
+miq.set_switch("M32_MIN_TB", 100)  # the 16-token kernel's scratch for 40 tokens, no workspace
+assert run("i8_gemm", small, 40)[1] == ["m16z_kernel"]
+miq.set_switch("M32_MIN_TB", miq.SWITCH_DEFAULT)
+fake.fake_capturing(1)
+for fn, pre in (("i8_gemm", []), ("i8_gemv_multi", []), ("quant_gemm", ["xq_kernel"]), ("quant_gemm_multi", ["xq_kernel"])):
+    assert run(fn, small, 40)[:2] == (OK, pre + ["m16z_kernel"]), (fn, run(fn, small, 40))
+assert run("i8_gemm", large, 512)[:2] == (UNSUPPORTED, [])
+fake.fake_capturing(0)
+assert run("quant_gemm", small, 40)[:2] == (OK, ["pf_quant_kernel", "pf16_kernel"])
+fake.fake_capturing(1)
+assert run("quant_gemm", small, 40)[:2] == (OK, ["pf_quant_kernel", "pf16_kernel"])
+""")

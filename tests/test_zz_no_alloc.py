@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
-Q4_K, Q5_K, Q6_K = 12, 13, 14
+Q8_0, Q4_K, Q5_K, Q6_K = 8, 12, 13, 14
 
 
 def _case(miq, dev, qt, N, K, TB, seed):
@@ -42,6 +42,22 @@ def test_noalloc_cu_resident_k_parts(miq, dev, switch):
         print(f"noalloc cu-form qt={qt} N={N} K={K} TB={TB}", flush=True)
         ref, got = _case(miq, dev, qt, N, K, TB, seed)
         assert np.array_equal(ref.view(np.uint32), got.view(np.uint32)), (qt, N, K, TB)
+
+
+@pytest.mark.parametrize("qt,N,K,TB", [(Q4_K, 17408, 5120, 40), (Q8_0, 5120, 5120, 20), (Q8_0, 5120, 5120, 130)])
+def test_noalloc_where_i8_gemm_takes_another_kernel(miq, oracle, dev, qt, N, K, TB):
+    """below 48 tokens miq_i8_gemm_noalloc stays on the 16-token kernel where
+    miq_i8_gemm takes a prefill kernel, and from there on Q8_0 runs without K
+    slices: both within the per-output bound of the oracle"""
+    from conftest import assert_elem, elem_bound
+    print(f"noalloc qt={qt} N={N} K={K} TB={TB}", flush=True)
+    rng = np.random.default_rng(TB)  # as _case draws them
+    wq = miq.quantize_rows(qt, (rng.standard_normal((N, K)) * 0.02).astype(np.float32))
+    x = rng.standard_normal((TB, K)).astype(np.float32)
+    a = oracle.xq(x)
+    exp, bound = oracle.gemm(qt, wq, K, N, a), elem_bound(oracle, qt, wq, K, a, 1.0)
+    for got in _case(miq, dev, qt, N, K, TB, TB):
+        assert_elem(got, exp, bound)
 
 
 def test_noalloc_refuses_prefill(miq, dev, switch):
