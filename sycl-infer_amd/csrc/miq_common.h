@@ -28,6 +28,21 @@ __host__ __device__ constexpr int block_bytes(uint32_t type) {
 // values per block
 __host__ __device__ constexpr int block_values(uint32_t type) { return type == MIQ_TYPE_Q8_0 ? 32 : 256; }
 
+// Arrival counters of a tile whose workgroups share an XCD, so that its partial
+// sums meet in that XCD's L2: a byte per XCD, so that the last to arrive sees
+// whether they do.  Workgroups of one blockIdx % 8 share an XCD, but not always
+// XCD blockIdx % 8: once a process has used several streams, whole launches of a
+// queue start at another XCD (all by the same offset in every launch measured, up
+// to five streams side by side), and stay so.  At most 255 workgroups per tile.
+// `astray` (a test): 1 in a workgroup that takes itself for one on another XCD.
+__device__ __forceinline__ uint64_t xcd_arrival(uint32_t astray) {
+    return 1ull << (8 * ((__builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) ^ astray) & 7));  // HW_REG_XCC_ID
+}
+__device__ __forceinline__ uint32_t xcd_arrived(uint64_t c) {
+    const uint64_t m = 0x00FF00FF00FF00FFull;
+    return (uint32_t)((((c & m) + ((c >> 8) & m)) * 0x0001000100010001ull) >> 48);
+}
+
 // Error plumbing shared by the entry points (miq_capi.hip).
 void set_error(const char *fmt, ...);
 int check_launch(const char *what);

@@ -159,19 +159,20 @@ __device__ __forceinline__ void wload(typename WOf<TYPE>::T &W, __amdgpu_buffer_
 // the whole slice land in registers while the staging completes.  The fold
 // then waits for each K step's own loads only.
 //
-// Slices of one tile run on one XCD (blockIdx % 8 == XCD, the dispatcher's
-// placement): blockIdx = 8 * (tile / 8 * S + slice) + tile % 8.  With one
+// Slices of one tile run on one XCD (the dispatcher deals workgroups to the XCDs
+// by blockIdx % 8): blockIdx = 8 * (tile / 8 * S + slice) + tile % 8.  With one
 // slice the tile is written directly; otherwise each slice leaves its partial
 // in the split-K scratch, and the last slice to arrive (arrival counter) sums
 // the S partials in slice order -- deterministic whatever the arrival order --
 // applies alpha and the residual and re-arms the counter.  The partials meet
 // in the XCD's L2 (stores drained before the arrival is counted, L1-bypassing
-// loads).  A workgroup that finds itself on another XCD (HW_REG_XCC_ID) uses
-// agent-scope fences and marks the counter so the reducer fences too.  That
-// covers a launch whose workgroups are all shifted to other XCDs, and a
-// misplaced slice that a well-placed one reduces; it does not cover a misplaced
-// last slice of a tile whose others are in place (they wrote nothing back past
-// their L2).  The dispatcher's round-robin placement produces neither.
+// loads).  A workgroup that finds itself on another XCD than blockIdx % 8
+// (HW_REG_XCC_ID) uses agent-scope fences and marks the counter so the reducer
+// fences too.  That covers a launch whose workgroups are all shifted by the same
+// number of XCDs (see xcd_arrival), and a misplaced slice that a well-placed one
+// reduces; it does not cover a misplaced last slice of a tile whose others are in
+// place (they wrote nothing back past their L2), which the dispatcher does not
+// produce.
 constexpr size_t kZSlotX = 8 * 512;    // codes of one K step: [group][h][token][8 B]
 constexpr size_t kZSlotM = 8 * 16 * 4; // one fp32 per (group, token)
 constexpr int kZXcd = 8;

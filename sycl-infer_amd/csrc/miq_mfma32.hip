@@ -51,7 +51,7 @@ struct M32Args {
     int nt, T;      // row tiles, tiles
     int S;          // K slices per tile
     float *part;    // [tile][slice][8][256 threads][4] partial sums (S > 1)
-    uint32_t *cnt;  // [tile] arrival counters, zero between launches
+    uint64_t *cnt;  // [tile] arrival counters (xcd_arrival), zero between launches
     int astray;     // a test: every second slice takes itself for one on another XCD
 };
 
@@ -243,7 +243,7 @@ __global__ __launch_bounds__(256, 2) void mfma32_kernel(M32Args A) {
     constexpr bool DOTS = FORM == kM32Dots;
     extern __shared__ __align__(16) uint8_t lds_raw[];
     M32Lds &L = *reinterpret_cast<M32Lds *>(lds_raw);
-    // Slices of one tile run on one XCD (blockIdx % 8, the dispatcher's placement):
+    // Slices of one tile run on one XCD (the dispatcher deals by blockIdx % 8):
     // blockIdx = 8 * (tile / 8 * S + slice) + tile % 8.
     int slice = 0, tile = blockIdx.x;
     if constexpr (FORM == kM32Sliced) {
@@ -392,49 +392,41 @@ sum_steps:
         // result does not depend on timing); one that finds every other one
         // arrived keeps its sums in registers.  The partials meet in the XCD's
         // L2 (stores drained before the arrival is counted, L1-bypassing
-        // loads).  A workgroup on another XCD than expected (HW_REG_XCC_ID; the
-        // dispatcher places none there) writes its partial back past its L2 and
-        // marks the counter so that the reducer drops stale lines first; where
-        // it is itself the last, it cannot see the others' partials and computes
-        // the whole tile instead, in one sum.
+        // loads).  Where the slices turn out to be on several XCDs (the dispatcher
+        // does not do that) their partials are of no use, and the last to arrive
+        // computes the whole tile instead, in one sum.
         __shared__ int lflag;
-        constexpr uint32_t kFar = 1u << 20;
         v4f32 *P = reinterpret_cast<v4f32 *>(A.part) + (size_t)tile * A.S * 2048 + threadIdx.x;
-        uint32_t *cnt = A.cnt + tile;
-        const bool far = (__builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 15) != (uint32_t)(blockIdx.x & 7) ||
-                         (A.astray && (slice & 1));
-        if (threadIdx.x == 0) {
-            const uint32_t prev = __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            lflag = (prev & (kFar - 1)) == (uint32_t)(A.S - 1) ? 1 + (prev >= kFar) : 0;
-        }
+        uint64_t *cnt = A.cnt + tile;
+        const uint64_t one = xcd_arrival((uint32_t)(A.astray & slice)), others = one * (uint32_t)(A.S - 1);
+        if (threadIdx.x == 0)
+            lflag = __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == others;
         __syncthreads();
         int fl = __builtin_amdgcn_readfirstlane(lflag);
         const bool own = fl;
         if (own) {
-            if (threadIdx.x == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (threadIdx.x == 0) __hip_atomic_store(cnt, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else {
 #pragma unroll
             for (int i = 0; i < 8; i++)
                 P[((size_t)slice * 8 + i) * 256] = v4f32{acc[i >> 2][4 * (i & 3)], acc[i >> 2][4 * (i & 3) + 1], acc[i >> 2][4 * (i & 3) + 2], acc[i >> 2][4 * (i & 3) + 3]};
-            if (far) __threadfence();
             __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
             if (threadIdx.x == 0) {
-                const uint32_t prev = __hip_atomic_fetch_add(cnt, far ? 1u + kFar : 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                const bool last = (prev & (kFar - 1)) == (uint32_t)(A.S - 1);
-                if (last) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                lflag = last ? 1 + (prev >= kFar) : 0;
+                const uint64_t prev = __hip_atomic_fetch_add(cnt, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const bool last = xcd_arrived(prev) == (uint32_t)(A.S - 1);
+                if (last) __hip_atomic_store(cnt, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                lflag = last ? 1 + (prev != others) : 0;
             }
             __syncthreads();
             fl = __builtin_amdgcn_readfirstlane(lflag);
         }
         if (!fl) return;
-        if (far) {
+        if (fl == 2) {
             kb0 = 0;
             nkb = steps;
             goto sum_steps;
         }
-        if (fl == 2) __threadfence();
         v16f sum[2] = {};
         const __amdgpu_buffer_rsrc_t rp = make_rsrc(reinterpret_cast<v4f32 *>(A.part) + (size_t)tile * A.S * 2048, (uint32_t)A.S * 32768u);
         for (int k = 0; k < A.S; k++) {
@@ -493,7 +485,7 @@ bool mfma32_fills(const miq_seg *s, int TB) {
 // tiles of 20 steps); sliced 25 us at 48, 31 at 128 and 52 at 333.
 static int m32_slices(const miq_seg *s, int TB, int n_cu) {
     const int T = ((s->n_rows + kBN - 1) / kBN) * ((TB + kBM - 1) / kBM), nkb = s->K / 256;
-    const int S = 2 * n_cu / T, most = nkb / 4;
+    const int S = 2 * n_cu / T, most = nkb / 4 < 255 ? nkb / 4 : 255;  // 255: xcd_arrival
     return S < 1 || most < 1 ? 1 : S < most ? S : most;
 }
 
@@ -541,7 +533,9 @@ int launch_mfma32(hipStream_t stream, const miq_seg *s, int TB, int32_t *dots) {
     A.S = dots ? 1 : m32_slices(s, TB, n_cu);
     // no scratch for the partials (a stream that captures a graph or has none of
     // its own, miq_i8_gemm_noalloc): unsliced
-    if (A.S > 1 && scratch_get(stream, (size_t)A.T * A.S * 32768, A.T, &A.part, &A.cnt) != MIQ_OK) A.S = 1;
+    uint32_t *cnt = nullptr;  // 8-byte counters, two of the scratch's 4-byte ones each
+    if (A.S > 1 && scratch_get(stream, (size_t)A.T * A.S * 32768, 2 * (size_t)A.T, &A.part, &cnt) != MIQ_OK) A.S = 1;
+    A.cnt = reinterpret_cast<uint64_t *>(cnt);
     A.astray = sw(kSwXcdAstray);
     const M32Form form = dots ? kM32Dots : A.S > 1 ? kM32Sliced : kM32Whole;
     const dim3 grid((unsigned)(form == kM32Sliced ? (A.T + 7) / 8 * 8 * A.S : A.T));

@@ -101,7 +101,7 @@ struct PfArgs {
     int mt;        // token tiles
     int nseg;
     float *part;   // per matrix [2 * workgroups] slots of [2*TT][512 threads][4] partial sums (stream-K)
-    uint32_t *cnt; // per matrix [tile] arrival counters, zero between launches
+    uint64_t *cnt; // per matrix [tile] arrival counters (xcd_arrival where xmap), zero between launches
     int32_t *dots; // parity form: [TB][n_rows][K/32] MFMA group results
     int astray;    // a test: every second workgroup of an XCD takes itself for one on another
     PfSeg seg[kPfSegs];
@@ -744,7 +744,7 @@ __global__ __launch_bounds__(kPT, 2) void pf16_kernel(PfArgs A) {
     // the next one's tiles.  Tile t is row tile t / mt, token tile t % mt, so the token
     // tiles of a row tile are neighbours and read its weights from L2.
     // `rounds` data-parallel rounds: in round k workgroup w takes tile
-    // k*P + (P/8)*(w % 8) + w/8, i.e. each XCD (blockIdx % 8) a run of
+    // k*P + (P/8)*(w % 8) + w/8, i.e. each XCD (dealt by blockIdx % 8) a run of
     // consecutive tiles; tiles past T are skipped.  The remaining `sk` tiles
     // are then split along K over all workgroups (stream-K): XCD x owns sk
     // tiles [x*sk/G, (x+1)*sk/G) and cuts their K blocks into P/G equal
@@ -753,12 +753,9 @@ __global__ __launch_bounds__(kPT, 2) void pf16_kernel(PfArgs A) {
     // for the tile it starts in, 2v+1 for the one it ends in), and the last
     // contributor to arrive adds the partials in range order (the result does
     // not depend on timing) and stores.  With G == 1 the partials go through
-    // memory, else those of a tile stay in their XCD's L2.  A workgroup that finds
-    // itself on another XCD than blockIdx % 8 (the dispatcher places none there)
-    // writes its partial back past its L2 and marks the counter so that the
-    // reducer drops stale lines first; where it is itself the last to arrive, it
-    // cannot see the others' partials and computes the whole tile, in one sum.
-    constexpr uint32_t kFar = 1u << 20;
+    // memory, else those of a tile stay in their XCD's L2; where its ranges turn
+    // out to be on several XCDs (the dispatcher does not do that) they are of no
+    // use, and the last to arrive computes the whole tile, in one sum.
     constexpr int kPart = 2 * TT * kPT;  // f4 of one partial tile
     const int w = blockIdx.x;
     for (int si = 0; si < A.nseg; si++) {
@@ -770,7 +767,7 @@ __global__ __launch_bounds__(kPT, 2) void pf16_kernel(PfArgs A) {
     const bool xmap = S.xmap;
     const int G = xmap ? 8 : 1, x = xmap ? w % 8 : 0, Pg = P / G, vl = xmap ? w / 8 : w;
     f4 *part = reinterpret_cast<f4 *>(A.part) + (size_t)S.poff * kPart;
-    uint32_t *cnt = A.cnt + S.coff;
+    uint64_t *cnt = A.cnt + S.coff;
     // XCD x's tiles [tx0, tx0 + ntx): the first sk % G XCDs hold one more; range u of
     // its ntx * nkb blocks starts at u*rq + min(u, rr) (the first rr ranges hold one more)
     const int ntx = sk / G + (x < sk % G), tx0 = F + x * (sk / G) + (x < sk % G ? x : sk % G);
@@ -826,44 +823,39 @@ __global__ __launch_bounds__(kPT, 2) void pf16_kernel(PfArgs A) {
         const int v_lo = owner(tb0), v_hi = owner(tb1 - 1);
         int n_contrib = 0;  // ranges of the tile that hold a block (with few blocks some are empty)
         for (int u = v_lo; u <= v_hi; u++) n_contrib += rstart(u) < rstart(u + 1);
-        const bool astray = xmap && ((__builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 15) != (uint32_t)x ||  // HW_REG_XCC_ID
-                                     (A.astray && (vl & 1)));
-        const bool far = !xmap || astray;
+        const uint64_t one = xmap ? xcd_arrival((uint32_t)(A.astray & vl)) : 1, others = one * (uint32_t)(n_contrib - 1);
         // A range that finds every other one arrived keeps its sums in registers.
-        if (tid == 0) {
-            const uint32_t prev = __hip_atomic_load(cnt + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            lflag = (prev & (kFar - 1)) == (uint32_t)(n_contrib - 1) ? 1 + (prev >= kFar) : 0;
-        }
+        if (tid == 0)
+            lflag = __hip_atomic_load(cnt + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == others;
         __syncthreads();
         int fl = __builtin_amdgcn_readfirstlane(lflag);
         const bool own = fl;
         if (own) {
-            if (tid == 0) __hip_atomic_store(cnt + t, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (tid == 0) __hip_atomic_store(cnt + t, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else {
             f4 *mine = part + (size_t)(2 * v + (head ? 0 : 1)) * kPart + tid;
 #pragma unroll
             for (int a = 0; a < 2; a++)
 #pragma unroll
                 for (int c = 0; c < TT; c++) mine[(a * TT + c) * kPT] = acc[a][c];
-            if (far) __threadfence();  // a reader on another XCD: write the partial back past the L2
+            if (!xmap) __threadfence();  // a reader on any XCD: write the partial back past the L2
             __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
             if (tid == 0) {
-                const uint32_t prev = __hip_atomic_fetch_add(cnt + t, far ? 1u + kFar : 1u, __ATOMIC_RELAXED,
-                                                             __HIP_MEMORY_SCOPE_AGENT);
-                const int last = (prev & (kFar - 1)) == (uint32_t)(n_contrib - 1);
-                if (last) __hip_atomic_store(cnt + t, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                lflag = last ? 1 + (prev >= kFar) : 0;
+                const uint64_t prev = __hip_atomic_fetch_add(cnt + t, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const bool last = prev == others || (xmap && xcd_arrived(prev) == (uint32_t)(n_contrib - 1));
+                if (last) __hip_atomic_store(cnt + t, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                lflag = last ? 1 + (prev != others) : 0;
             }
             __syncthreads();
             fl = __builtin_amdgcn_readfirstlane(lflag);
         }
         if (!fl) continue;
-        if (__builtin_expect(astray, 0)) {
+        if (__builtin_expect(fl == 2, 0)) {
             b0 += kAgain;
             continue;
         }
-        if (fl == 2 || far) __threadfence();  // some partial crossed XCDs: drop stale L2 lines first
+        if (!xmap) __threadfence();  // drop stale L2 lines first
         f4 sum[2][TT];
 #pragma unroll
         for (int a = 0; a < 2; a++)
@@ -1073,11 +1065,11 @@ static int launch(hipStream_t stream, const miq_seg *segs, int n_segs, int TB, i
     void *ws = nullptr, *cw = nullptr;
     *no_ws = true;
     if (const int rc = workspace_get(stream, kWsPrefill, rec_bytes + max_slots * slot_bytes, &ws)) return rc;
-    if (const int rc = workspace_get(stream, kWsPrefillCnt, (size_t)max_tiles * 4, &cw, true)) return rc;
+    if (const int rc = workspace_get(stream, kWsPrefillCnt, (size_t)max_tiles * 8, &cw, true)) return rc;
     *no_ws = false;
     A.rec = reinterpret_cast<const uint8_t *>(ws);
     A.part = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(ws) + rec_bytes);
-    A.cnt = reinterpret_cast<uint32_t *>(cw);
+    A.cnt = reinterpret_cast<uint64_t *>(cw);
     int nb = (int)nkb, tb = TB, stride = s->x_stride;
     uint8_t *rec = reinterpret_cast<uint8_t *>(ws);
     hipError_t e;

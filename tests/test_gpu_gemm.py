@@ -498,9 +498,8 @@ def test_gemm_prefill_int8_slices(miq, oracle, dev, qt, TB, N, K, switch):
                                        (Q6_K, 256, 3000, 1024)])
 def test_prefill_partials_across_xcds(miq, oracle, dev, qt, TB, N, K, switch):
     """Both prefill GEMMs where every second workgroup that shares a tile takes itself
-    for one on another XCD (XCD_ASTRAY): its partial goes through memory, and where it
-    is the last it computes the tile again.  Within the per-output bound in every run,
-    with the normal placement's bits back afterwards."""
+    for one on another XCD (XCD_ASTRAY): the last of the tile computes it again.  Within
+    the per-output bound in every run, with the normal placement's bits back afterwards."""
     import torch
     print(f"prefill across XCDs qt={qt} TB={TB} N={N} K={K}", flush=True)
     switch("PREFILL_FP16", "2")
@@ -531,6 +530,37 @@ def test_prefill_partials_across_xcds(miq, oracle, dev, qt, TB, N, K, switch):
     assert differ  # some tile was computed in one sum
     switch("XCD_ASTRAY", "0")
     assert np.array_equal(run().view(np.uint32), normal.view(np.uint32))
+
+
+@pytest.mark.parametrize("qt,TB,N,K", [(Q8_0, 200, 5120, 2560), (Q4_K, 77, 4096, 4096), (Q5_K, 200, 7168, 2048), (Q6_K, 130, 2048, 5120),
+                                       (Q4_K, 16, 4096, 4096), (Q6_K, 16, 40960, 5120)])
+def test_gemm_bits_after_streams_overlapped(miq, oracle, dev, qt, TB, N, K, switch):
+    """Once several streams have run side by side, a queue's workgroups all start at
+    another XCD than before: the same bits on every stream, one at a time."""
+    import torch
+    print(f"bits after streams overlapped qt={qt} TB={TB} N={N} K={K}", flush=True)
+    switch("PREFILL_FP16", "2")
+    wq = weights(miq, qt, N, K, seed=TB)
+    x = np.random.default_rng(TB + K).standard_normal((TB, K)).astype(np.float32)
+    wd, act = to_dev(wq, dev), miq.xq(to_dev(x, dev))
+    streams = [torch.cuda.default_stream()] + [torch.cuda.Stream() for _ in range(5)]
+    busy = [torch.zeros(1 << 22, device=dev) for _ in streams]
+    torch.cuda.synchronize()
+    got = []
+    for _ in range(2):
+        for s in streams:
+            with torch.cuda.stream(s):
+                out = torch.full((TB, N), float("nan"), dtype=torch.float32, device=dev)
+                miq.i8_gemm(miq.make_seg(wd, qt, K, N, act, out, N), TB)
+                torch.cuda.synchronize()
+            got.append(out.cpu().numpy())
+        for i in range(120):
+            with torch.cuda.stream(streams[i % len(streams)]):
+                busy[i % len(streams)].add_(1.0)
+        torch.cuda.synchronize()
+    assert all(np.array_equal(g.view(np.uint32), got[0].view(np.uint32)) for g in got[1:])
+    a = oracle.xq(x)
+    assert_elem(got[0], oracle.gemm(qt, wq, K, N, a), elem_bound(oracle, qt, wq, K, a, 1.0))
 
 
 @pytest.mark.parametrize("TB,N,K", [(200, 5120, 2560), (64, 1024, 5120)])
