@@ -170,8 +170,8 @@ int miq_group_dots(hipStream_t stream, const void *w, uint32_t type, int K, int 
 
 /* Set a tuning switch (an A/B form of a kernel choice) by name: M32_MIN_TB,
  * GEMV_MAX_TB, PREFILL_FP16, FUSED_QUANT, M16_WAVES, M16_FORM, MOE_GRP,
- * M32_FILL, and XCD_ASTRAY (a test of the prefill GEMMs: workgroups that take
- * themselves for misplaced).  Each
+ * M32_FILL, and XCD_ASTRAY (a test: workgroups that share a tile take themselves
+ * for ones on several XCDs).  Each
  * starts from the environment variable MIQ_<name> (read once per process) or
  * its default; value INT_MIN restores that.  Every form gives results within
  * the same bounds; the defaults are the measured fastest.  The reference

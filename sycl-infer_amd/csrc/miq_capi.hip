@@ -50,7 +50,7 @@ namespace {
 struct Scratch {
     float *part = nullptr;
     size_t part_bytes = 0;
-    uint32_t *cnt = nullptr;
+    uint64_t *cnt = nullptr;
     size_t n_cnt = 0;
 };
 constexpr int kMaxDevices = 64;
@@ -94,7 +94,7 @@ int may_grow(hipStream_t stream, const char *what, size_t have, size_t want) {
 // keep the last call's contents.  Calls that overlap on one device race.
 constexpr size_t kStaticPartBytes = (size_t)16 << 20;
 constexpr size_t kStaticCnt = (size_t)64 << 10;
-static __device__ __align__(256) uint8_t scratch[kStaticPartBytes + kStaticCnt * sizeof(uint32_t)];
+static __device__ __align__(256) uint8_t scratch[kStaticPartBytes + kStaticCnt * sizeof(uint64_t)];
 
 namespace {
 uint8_t *g_static_ptr[kMaxDevices];
@@ -113,7 +113,7 @@ struct StaticMode {
 
 bool static_scratch_mode() { return g_static_mode; }
 
-static int static_scratch_get(hipStream_t stream, size_t part_bytes, size_t n_cnt, float **part, uint32_t **cnt) {
+static int static_scratch_get(hipStream_t stream, size_t part_bytes, size_t n_cnt, float **part, uint64_t **cnt) {
     if (part_bytes > kStaticPartBytes || n_cnt > kStaticCnt) {
         set_error("miq_i8_gemm_noalloc: the shape needs %zu bytes of partials and %zu counters, beyond the static "
                   "scratch (%zu bytes, %zu counters)", part_bytes, n_cnt, kStaticPartBytes, kStaticCnt);
@@ -141,13 +141,13 @@ static int static_scratch_get(hipStream_t stream, size_t part_bytes, size_t n_cn
         }
         if (cs == hipStreamCaptureStatusNone) {
             hipLaunchKernelGGL(zero_u32_kernel, dim3(64), dim3(256), 0, stream,
-                               reinterpret_cast<uint32_t *>(p + kStaticPartBytes), kStaticCnt);
+                               reinterpret_cast<uint32_t *>(p + kStaticPartBytes), 2 * kStaticCnt);
             if (check_launch("miq_i8_gemm_noalloc: clearing the static counters") != MIQ_OK) return MIQ_EHIP;
         }
         g_static_ptr[dev] = p;
     }
     *part = reinterpret_cast<float *>(g_static_ptr[dev]);
-    *cnt = reinterpret_cast<uint32_t *>(g_static_ptr[dev] + kStaticPartBytes);
+    *cnt = reinterpret_cast<uint64_t *>(g_static_ptr[dev] + kStaticPartBytes);
     return MIQ_OK;
 }
 
@@ -174,16 +174,16 @@ static int grow_scratch(Scratch &s, hipStream_t stream, size_t part_bytes, size_
         s.part_bytes = want;
     }
     if (s.n_cnt < n_cnt) {
-        if (const int rc = may_grow(stream, "split-K counters", s.n_cnt * 4, n_cnt * 4)) return rc;
+        if (const int rc = may_grow(stream, "split-K counters", s.n_cnt * 8, n_cnt * 8)) return rc;
         const size_t want = n_cnt + n_cnt / 2 + 64;
-        uint32_t *nc = nullptr;
-        if (!device_alloc((void **)&nc, want * sizeof(uint32_t))) {
+        uint64_t *nc = nullptr;
+        if (!device_alloc((void **)&nc, want * sizeof(uint64_t))) {
             set_error("split-K scratch: counter allocation failed");
             return MIQ_EHIP;
         }
         // cleared on the caller's stream, so the clear is ordered before the
         // kernel that reads the counters whatever kind of stream it is
-        hipLaunchKernelGGL(zero_u32_kernel, dim3(64), dim3(256), 0, stream, nc, want);
+        hipLaunchKernelGGL(zero_u32_kernel, dim3(64), dim3(256), 0, stream, reinterpret_cast<uint32_t *>(nc), 2 * want);
         if (check_launch("split-K scratch: clearing the counters") != MIQ_OK) return MIQ_EHIP;
         if (s.cnt) g_retired.push_back(s.cnt);
         s.cnt = nc;
@@ -235,7 +235,7 @@ static int own_scratch(hipStream_t stream, OwnSlot *slots, OwnSlot **out) {
     return MIQ_OK;
 }
 
-int scratch_get(hipStream_t stream, size_t part_bytes, size_t n_cnt, float **part, uint32_t **cnt) {
+int scratch_get(hipStream_t stream, size_t part_bytes, size_t n_cnt, float **part, uint64_t **cnt) {
     if (g_static_mode && !g_own_mode) return static_scratch_get(stream, part_bytes, n_cnt, part, cnt);
     int dev = 0;
     if (current_device(&dev) != MIQ_OK) return MIQ_EHIP;

@@ -28,19 +28,33 @@ __host__ __device__ constexpr int block_bytes(uint32_t type) {
 // values per block
 __host__ __device__ constexpr int block_values(uint32_t type) { return type == MIQ_TYPE_Q8_0 ? 32 : 256; }
 
-// Arrival counters of a tile whose workgroups share an XCD, so that its partial
-// sums meet in that XCD's L2: a byte per XCD, so that the last to arrive sees
-// whether they do.  Workgroups of one blockIdx % 8 share an XCD, but not always
-// XCD blockIdx % 8: once a process has used several streams, whole launches of a
-// queue start at another XCD (all by the same offset in every launch measured, up
-// to five streams side by side), and stay so.  At most 255 workgroups per tile.
-// `astray` (a test): 1 in a workgroup that takes itself for one on another XCD.
-__device__ __forceinline__ uint64_t xcd_arrival(uint32_t astray) {
-    return 1ull << (8 * ((__builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) ^ astray) & 7));  // HW_REG_XCC_ID
+// Partial sums of a tile that several workgroups share.  Workgroups of one
+// blockIdx % 8 share an XCD, so the partials of a tile laid out that way meet in
+// one L2, but not always XCD blockIdx % 8's: once a process has used several
+// streams, a queue's launches start at another XCD (all workgroups by the same
+// offset in every launch measured, five streams side by side) and stay so.  So
+// no workgroup expects an XCD: each drains its partial and adds xcd_arrival() to
+// the tile's counter, and the last to arrive learns whether everyone was on its
+// XCD.  Then it reads the partials from L2.  Else, which the dispatcher does not
+// produce, a prefill GEMM computes the tile again, and the 16-token kernel, whose
+// partials are written through (agent scope), reads them past the L2.  Dearer: a
+// fence per workgroup (40 to 200 us a launch), agent scope on both sides (up to
+// 9 us where 14 slices meet, Q8_0 4096 x 14336 at 40 tokens 44 -> 53), and for the
+// fp16 GEMM the write-through (17408 x 5120 at 128 tokens 53.9 -> 57.4).
+constexpr int kAgentScope = 16;  // last operand of a buffer access: the sc1 bit
+constexpr int kL2 = 1;           // and sc0, past the CU's L1
+// The counter holds the number of arrivals (at most 65535) and the sums of their
+// XCDs' numbers and of the squares of those, so it is n times one arrival's only
+// if all n were on that one's XCD.  `astray` (a test): 1 in a workgroup that takes
+// itself for one on another XCD.
+constexpr uint64_t kArrivals = 0xFFFF;
+__device__ __forceinline__ uint64_t xcd_arrival(int astray) {
+    const uint32_t x = (__builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) ^ (uint32_t)astray) & 15;  // HW_REG_XCC_ID
+    return 1 | (uint64_t)x << 16 | (uint64_t)(x * x) << 40;
 }
-__device__ __forceinline__ uint32_t xcd_arrived(uint64_t c) {
-    const uint64_t m = 0x00FF00FF00FF00FFull;
-    return (uint32_t)((((c & m) + ((c >> 8) & m)) * 0x0001000100010001ull) >> 48);
+// What an arrival (mine) finds, of n: 0 it is not the last, 1 all were on its XCD, 2 not all.
+__device__ __forceinline__ int xcd_last(uint64_t before, uint64_t mine, uint32_t n) {
+    return (before & kArrivals) != n - 1 ? 0 : before == mine * (n - 1) ? 1 : 2;
 }
 
 // Error plumbing shared by the entry points (miq_capi.hip).

@@ -8,7 +8,7 @@ namespace miq {
 // Per-device split-K scratch (partial tiles + zeroed arrival counters).  Grown
 // only outside stream capture (MIQ_UNSUPPORTED if `stream` captures and the
 // buffers are too small).
-int scratch_get(hipStream_t stream, size_t part_bytes, size_t n_cnt, float **part, uint32_t **cnt);
+int scratch_get(hipStream_t stream, size_t part_bytes, size_t n_cnt, float **part, uint64_t **cnt);
 // While one with on == true lives, this thread's scratch_get() gives buffers of
 // the stream's own, or MIQ_UNSUPPORTED where there are none.
 struct OwnScratch {

@@ -159,24 +159,22 @@ __device__ __forceinline__ void wload(typename WOf<TYPE>::T &W, __amdgpu_buffer_
 // the whole slice land in registers while the staging completes.  The fold
 // then waits for each K step's own loads only.
 //
-// Slices of one tile run on one XCD (the dispatcher deals workgroups to the XCDs
-// by blockIdx % 8): blockIdx = 8 * (tile / 8 * S + slice) + tile % 8.  With one
-// slice the tile is written directly; otherwise each slice leaves its partial
-// in the split-K scratch, and the last slice to arrive (arrival counter) sums
-// the S partials in slice order -- deterministic whatever the arrival order --
-// applies alpha and the residual and re-arms the counter.  The partials meet
-// in the XCD's L2 (stores drained before the arrival is counted, L1-bypassing
-// loads).  A workgroup that finds itself on another XCD than blockIdx % 8
-// (HW_REG_XCC_ID) uses agent-scope fences and marks the counter so the reducer
-// fences too.  That covers a launch whose workgroups are all shifted by the same
-// number of XCDs (see xcd_arrival), and a misplaced slice that a well-placed one
-// reduces; it does not cover a misplaced last slice of a tile whose others are in
-// place (they wrote nothing back past their L2), which the dispatcher does not
-// produce.
+// blockIdx = 8 * (tile / 8 * S + slice) + tile % 8, so that the slices of one tile
+// run on one XCD (the dispatcher deals workgroups to the XCDs by blockIdx % 8).
+// With one slice the tile is written directly; otherwise each slice leaves its
+// partial in the split-K scratch, and the last slice to arrive (arrival counter)
+// sums the S partials in slice order -- deterministic whatever the arrival order --
+// applies alpha and the residual and re-arms the counter.  The partials are written
+// through to memory and read from the XCD's L2 where every slice was on this XCD,
+// else past it (see xcd_arrival); computing the tile again instead would need no
+// write-through, but its code costs the folds 2 to 12 % by its registers.  Against
+// partials left in L2: Q4_K 1024 x 5120, 8 tokens 11.8 -> 12.6 us,
+// Q6_K 1024 x 4096 16 tokens 12.2 -> 11.5 and Q8_0 1024 x 5120 64 tokens 18.2 -> 17.8
+// (a counter in 64 bits).
 constexpr size_t kZSlotX = 8 * 512;    // codes of one K step: [group][h][token][8 B]
 constexpr size_t kZSlotM = 8 * 16 * 4; // one fp32 per (group, token)
 constexpr int kZXcd = 8;
-constexpr uint32_t kZFar = 1u << 20;   // counter mark: a partial came from another XCD
+typedef uint32_t u4x __attribute__((ext_vector_type(4)));
 // K steps per slice at most (register budget of the weight operands)
 template <uint32_t TYPE> constexpr int z_ks() {
     return TYPE == MIQ_TYPE_Q8_0 ? 2 : TYPE == MIQ_TYPE_Q6_K ? 3 : TYPE == MIQ_TYPE_Q5_K ? 5 : 7;
@@ -214,7 +212,8 @@ struct ZArgs {
     int nkb;        // K steps per row (the last one partial for Q8_0 when K % 256 != 0)
     int nseg;
     float *part;    // partial tiles of every segment
-    uint32_t *cnt;  // arrival counters, zero between launches
+    uint64_t *cnt;  // arrival counters, zero between launches
+    int astray;     // a test: every second slice takes itself for one on another XCD
     ZSeg seg[kZSegs];
 };
 
@@ -441,7 +440,7 @@ __global__ __launch_bounds__(64 * NW, 16 / NW) void m16z_kernel(ZArgs P) {
     const int nkb = P.nkb;
     const int tt = tile / G.ngrp, rg = tile - tt * G.ngrp;
     float *const part = P.part + G.poff;
-    uint32_t *const cnt = P.cnt + G.coff;
+    uint64_t *const cnt = P.cnt + G.coff;
     const int kb0 = s * nkb / S, nb = (s + 1) * nkb / S - kb0;
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -594,40 +593,39 @@ __global__ __launch_bounds__(64 * NW, 16 / NW) void m16z_kernel(ZArgs P) {
         store(cv);
         return;
     }
-    const bool far = (__builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 15) != (uint32_t)x;  // HW_REG_XCC_ID
     constexpr int kTile = 256 * NW;  // fp32 outputs per tile
-    *reinterpret_cast<v4f *>(part + ((size_t)tile * S + s) * kTile + threadIdx.x * 4) = cv;
-    if (far) __threadfence();  // another XCD will read this partial: write it back past the L2
+    const __amdgpu_buffer_rsrc_t rp = make_rsrc(part, (uint32_t)((size_t)G.ntile * S * kTile * 4));
+    const uint32_t pbase = (uint32_t)((size_t)tile * S * kTile + threadIdx.x * 4) * 4;
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4x, cv), rp, pbase + (uint32_t)s * kTile * 4, 0, kAgentScope);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     if (threadIdx.x == 0) {
-        const uint32_t prev = __hip_atomic_fetch_add(cnt + tile, far ? 1u + kZFar : 1u, __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT);
-        const int last = (prev & (kZFar - 1)) == (uint32_t)(S - 1);
-        if (last) __hip_atomic_store(cnt + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        lflag = last ? 1 + (prev >= kZFar) : 0;
+        const uint64_t one = xcd_arrival(P.astray & s);
+        const uint64_t prev = __hip_atomic_fetch_add(cnt + tile, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        lflag = xcd_last(prev, one, (uint32_t)S);
+        if (lflag) __hip_atomic_store(cnt + tile, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
-    const int fl = lflag;
+    const int fl = __builtin_amdgcn_readfirstlane(lflag);
     if (!fl) return;
-    if (fl == 2 || far) __threadfence();  // some partial crossed XCDs: drop stale L2 lines first
-    // four partials in flight at a time, summed in slice order; glc: past this
-    // CU's L1 to the XCD's L2 where they met
-    const __amdgpu_buffer_rsrc_t rp = make_rsrc(part, (uint32_t)((size_t)G.ntile * S * kTile * 4));
-    const uint32_t pbase = (uint32_t)((size_t)tile * S * kTile + threadIdx.x * 4) * 4;
+    // four partials in flight at a time, summed in slice order
     v4f sum = {0, 0, 0, 0};
-    for (int p0 = 0; p0 < S; p0 += 4) {
-        v4f pv[4];
+    auto add = [&](auto scope) {
+        for (int p0 = 0; p0 < S; p0 += 4) {
+            v4f pv[4];
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const uint32_t off = p0 + k < S ? pbase + (uint32_t)(p0 + k) * kTile * 4 : 0xFFFFFFF0u;
-            pv[k] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rp, off, 0, 1));
+            for (int k = 0; k < 4; k++) {
+                const uint32_t off = p0 + k < S ? pbase + (uint32_t)(p0 + k) * kTile * 4 : 0xFFFFFFF0u;
+                pv[k] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rp, off, 0, decltype(scope)::value));
+            }
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) sum[v] += pv[k][v];
         }
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) sum[v] += pv[k][v];
-    }
+    };
+    if (fl == 1) add(std::integral_constant<int, kL2>{});
+    else add(std::integral_constant<int, kAgentScope>{});
     store(sum);
 }
 
@@ -642,8 +640,9 @@ __global__ __launch_bounds__(64 * NW, 16 / NW) void m16z_kernel(ZArgs P) {
 // ranges and stream their weight bytes with PD steps in flight.  A tile that
 // one wave covers completely is finished by that wave; the pieces of a tile
 // shared by waves meet in LDS and are added in wave order.  With KP > 1 the
-// parts of a tile meet in a global partial buffer (their CUs share an XCD),
-// the last to arrive adding them in part order.
+// parts of a tile meet in a global partial buffer, written and read at agent
+// scope (free here: 65536 x 8192 Q6_K 123 us either way), the last to arrive adding
+// them in part order.
 constexpr int kCWaves = 8;
 constexpr int kCMaxSteps = 20;                        // K steps of activation one CU holds
 constexpr size_t kCRedOff = kCMaxSteps * (kZSlotX + 3 * kZSlotM);
@@ -656,7 +655,7 @@ struct CArgs {
     int G;          // workgroups per K part
     int NT;         // 16-row tiles
     float *part;    // [NT][KP][256] fp32 (KP > 1)
-    uint32_t *cnt;  // [NT] arrival counters, zero between launches (KP > 1)
+    uint64_t *cnt;  // [NT] arrival counters, zero between launches (KP > 1)
 };
 
 template <uint32_t TYPE> constexpr int c_pd() {  // K steps in flight per wave
@@ -743,7 +742,6 @@ __global__ __launch_bounds__(64 * kCWaves, 1) void m16c_kernel(CArgs P) {
     __syncthreads();
 
     // ---- finishing a tile: C[token 4h+v][row col] for this K part
-    const bool far = (__builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 15) != (uint32_t)(b % 8);  // HW_REG_XCC_ID
     auto store = [&](int tile, const v4f &val) {
         const int row = tile * 16 + col;
 #pragma unroll
@@ -762,21 +760,16 @@ __global__ __launch_bounds__(64 * kCWaves, 1) void m16c_kernel(CArgs P) {
             store(tile, val);
             return;
         }
-        constexpr uint32_t kFar = 1u << 20;
-        *reinterpret_cast<v4f *>(P.part + ((size_t)tile * P.KP + kp) * 256 + lane * 4) = val;
-        if (far) __threadfence();  // misplaced: see the split-K form above for what this covers
-        __builtin_amdgcn_s_waitcnt(0);
-        uint32_t prev = 0;
-        if (lane == 0) prev = __hip_atomic_fetch_add(P.cnt + tile, far ? 1u + kFar : 1u, __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT);
-        prev = __builtin_amdgcn_readfirstlane(prev);
-        if ((prev & (kFar - 1)) != (uint32_t)(P.KP - 1)) return;
-        if (lane == 0) __hip_atomic_store(P.cnt + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (prev >= kFar || far) __threadfence();
         const __amdgpu_buffer_rsrc_t rp = make_rsrc(P.part + (size_t)tile * P.KP * 256, (uint32_t)P.KP * 1024);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4x, val), rp, (uint32_t)(kp * 256 + lane * 4) * 4, 0, kAgentScope);
+        __builtin_amdgcn_s_waitcnt(0);
+        uint64_t prev = 0;
+        if (lane == 0) prev = __hip_atomic_fetch_add(P.cnt + tile, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (__builtin_amdgcn_readfirstlane((uint32_t)prev) != (uint32_t)(P.KP - 1)) return;
+        if (lane == 0) __hip_atomic_store(P.cnt + tile, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         v4f sum = {0, 0, 0, 0};
         for (int k = 0; k < P.KP; k++)
-            sum += __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rp, (uint32_t)(k * 256 + lane * 4) * 4, 0, 1));
+            sum += __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rp, (uint32_t)(k * 256 + lane * 4) * 4, 0, kAgentScope));
         store(tile, sum);
     };
 
@@ -915,6 +908,7 @@ template <uint32_t TYPE> static int launch_m16z(hipStream_t stream, const M16Arg
     const int nw = nw_set == 4 || nw_set == 8 ? nw_set : TYPE == MIQ_TYPE_Q4_K ? 8 : 4;
     ZArgs P{};
     P.a = A;
+    P.astray = sw(kSwXcdAstray);
     P.nkb = (A.K + 255) / 256;
     P.nseg = nseg;
     long nwg = 0;

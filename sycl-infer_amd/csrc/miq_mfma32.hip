@@ -26,6 +26,7 @@ typedef int v4i32 __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v4f32 __attribute__((ext_vector_type(4)));
+typedef uint32_t v4u32 __attribute__((ext_vector_type(4)));
 
 constexpr int kBM = 64;   // tokens per workgroup
 constexpr int kBN = 128;  // weight rows per workgroup
@@ -392,15 +393,13 @@ sum_steps:
         // result does not depend on timing); one that finds every other one
         // arrived keeps its sums in registers.  The partials meet in the XCD's
         // L2 (stores drained before the arrival is counted, L1-bypassing
-        // loads).  Where the slices turn out to be on several XCDs (the dispatcher
-        // does not do that) their partials are of no use, and the last to arrive
-        // computes the whole tile instead, in one sum.
+        // loads); where the slices were on several XCDs (see xcd_arrival), the last
+        // to arrive computes the whole tile instead, in one sum.
         __shared__ int lflag;
-        v4f32 *P = reinterpret_cast<v4f32 *>(A.part) + (size_t)tile * A.S * 2048 + threadIdx.x;
+        const __amdgpu_buffer_rsrc_t rp = make_rsrc(reinterpret_cast<v4f32 *>(A.part) + (size_t)tile * A.S * 2048, (uint32_t)A.S * 32768u);
         uint64_t *cnt = A.cnt + tile;
-        const uint64_t one = xcd_arrival((uint32_t)(A.astray & slice)), others = one * (uint32_t)(A.S - 1);
         if (threadIdx.x == 0)
-            lflag = __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == others;
+            lflag = xcd_last(__hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), xcd_arrival(A.astray & slice), (uint32_t)A.S) == 1;
         __syncthreads();
         int fl = __builtin_amdgcn_readfirstlane(lflag);
         const bool own = fl;
@@ -409,14 +408,16 @@ sum_steps:
         } else {
 #pragma unroll
             for (int i = 0; i < 8; i++)
-                P[((size_t)slice * 8 + i) * 256] = v4f32{acc[i >> 2][4 * (i & 3)], acc[i >> 2][4 * (i & 3) + 1], acc[i >> 2][4 * (i & 3) + 2], acc[i >> 2][4 * (i & 3) + 3]};
+                __builtin_amdgcn_raw_buffer_store_b128(
+                    __builtin_bit_cast(v4u32, v4f32{acc[i >> 2][4 * (i & 3)], acc[i >> 2][4 * (i & 3) + 1], acc[i >> 2][4 * (i & 3) + 2], acc[i >> 2][4 * (i & 3) + 3]}),
+                    rp, threadIdx.x * 16, (slice * 8 + i) * 4096, 0);
             __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
             if (threadIdx.x == 0) {
+                const uint64_t one = xcd_arrival(A.astray & slice);
                 const uint64_t prev = __hip_atomic_fetch_add(cnt, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                const bool last = xcd_arrived(prev) == (uint32_t)(A.S - 1);
-                if (last) __hip_atomic_store(cnt, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                lflag = last ? 1 + (prev != others) : 0;
+                lflag = xcd_last(prev, one, (uint32_t)A.S);
+                if (lflag) __hip_atomic_store(cnt, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             __syncthreads();
             fl = __builtin_amdgcn_readfirstlane(lflag);
@@ -428,7 +429,6 @@ sum_steps:
             goto sum_steps;
         }
         v16f sum[2] = {};
-        const __amdgpu_buffer_rsrc_t rp = make_rsrc(reinterpret_cast<v4f32 *>(A.part) + (size_t)tile * A.S * 2048, (uint32_t)A.S * 32768u);
         for (int k = 0; k < A.S; k++) {
             if (own && k == slice) {
 #pragma unroll
@@ -437,8 +437,7 @@ sum_steps:
             }
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                const v4f32 q = __builtin_bit_cast(v4f32, __builtin_amdgcn_raw_buffer_load_b128(
-                                                              rp, (uint32_t)(((k * 8 + i) * 256 + (int)threadIdx.x) * 16), 0, 1));
+                const v4f32 q = __builtin_bit_cast(v4f32, __builtin_amdgcn_raw_buffer_load_b128(rp, threadIdx.x * 16, (k * 8 + i) * 4096, 1));
 #pragma unroll
                 for (int v = 0; v < 4; v++) sum[i >> 2][4 * (i & 3) + v] += q[v];
             }
@@ -485,7 +484,7 @@ bool mfma32_fills(const miq_seg *s, int TB) {
 // tiles of 20 steps); sliced 25 us at 48, 31 at 128 and 52 at 333.
 static int m32_slices(const miq_seg *s, int TB, int n_cu) {
     const int T = ((s->n_rows + kBN - 1) / kBN) * ((TB + kBM - 1) / kBM), nkb = s->K / 256;
-    const int S = 2 * n_cu / T, most = nkb / 4 < 255 ? nkb / 4 : 255;  // 255: xcd_arrival
+    const int S = 2 * n_cu / T, most = nkb / 4;
     return S < 1 || most < 1 ? 1 : S < most ? S : most;
 }
 
@@ -533,9 +532,7 @@ int launch_mfma32(hipStream_t stream, const miq_seg *s, int TB, int32_t *dots) {
     A.S = dots ? 1 : m32_slices(s, TB, n_cu);
     // no scratch for the partials (a stream that captures a graph or has none of
     // its own, miq_i8_gemm_noalloc): unsliced
-    uint32_t *cnt = nullptr;  // 8-byte counters, two of the scratch's 4-byte ones each
-    if (A.S > 1 && scratch_get(stream, (size_t)A.T * A.S * 32768, 2 * (size_t)A.T, &A.part, &cnt) != MIQ_OK) A.S = 1;
-    A.cnt = reinterpret_cast<uint64_t *>(cnt);
+    if (A.S > 1 && scratch_get(stream, (size_t)A.T * A.S * 32768, A.T, &A.part, &A.cnt) != MIQ_OK) A.S = 1;
     A.astray = sw(kSwXcdAstray);
     const M32Form form = dots ? kM32Dots : A.S > 1 ? kM32Sliced : kM32Whole;
     const dim3 grid((unsigned)(form == kM32Sliced ? (A.T + 7) / 8 * 8 * A.S : A.T));

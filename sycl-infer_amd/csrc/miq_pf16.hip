@@ -101,7 +101,7 @@ struct PfArgs {
     int mt;        // token tiles
     int nseg;
     float *part;   // per matrix [2 * workgroups] slots of [2*TT][512 threads][4] partial sums (stream-K)
-    uint64_t *cnt; // per matrix [tile] arrival counters (xcd_arrival where xmap), zero between launches
+    uint64_t *cnt; // per matrix [tile] arrival counters (xcd_arrival), zero between launches
     int32_t *dots; // parity form: [TB][n_rows][K/32] MFMA group results
     int astray;    // a test: every second workgroup of an XCD takes itself for one on another
     PfSeg seg[kPfSegs];
@@ -753,9 +753,9 @@ __global__ __launch_bounds__(kPT, 2) void pf16_kernel(PfArgs A) {
     // for the tile it starts in, 2v+1 for the one it ends in), and the last
     // contributor to arrive adds the partials in range order (the result does
     // not depend on timing) and stores.  With G == 1 the partials go through
-    // memory, else those of a tile stay in their XCD's L2; where its ranges turn
-    // out to be on several XCDs (the dispatcher does not do that) they are of no
-    // use, and the last to arrive computes the whole tile, in one sum.
+    // memory, else those of a tile stay in their XCD's L2; where its ranges were on
+    // several XCDs all the same (see xcd_arrival), the last to arrive computes the
+    // whole tile, in one sum.
     constexpr int kPart = 2 * TT * kPT;  // f4 of one partial tile
     const int w = blockIdx.x;
     for (int si = 0; si < A.nseg; si++) {
@@ -823,10 +823,10 @@ __global__ __launch_bounds__(kPT, 2) void pf16_kernel(PfArgs A) {
         const int v_lo = owner(tb0), v_hi = owner(tb1 - 1);
         int n_contrib = 0;  // ranges of the tile that hold a block (with few blocks some are empty)
         for (int u = v_lo; u <= v_hi; u++) n_contrib += rstart(u) < rstart(u + 1);
-        const uint64_t one = xmap ? xcd_arrival((uint32_t)(A.astray & vl)) : 1, others = one * (uint32_t)(n_contrib - 1);
+        const uint64_t one = xmap ? xcd_arrival(A.astray & vl) : 1;
         // A range that finds every other one arrived keeps its sums in registers.
         if (tid == 0)
-            lflag = __hip_atomic_load(cnt + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == others;
+            lflag = xcd_last(__hip_atomic_load(cnt + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), one, (uint32_t)n_contrib) == 1;
         __syncthreads();
         int fl = __builtin_amdgcn_readfirstlane(lflag);
         const bool own = fl;
@@ -837,15 +837,15 @@ __global__ __launch_bounds__(kPT, 2) void pf16_kernel(PfArgs A) {
 #pragma unroll
             for (int a = 0; a < 2; a++)
 #pragma unroll
-                for (int c = 0; c < TT; c++) mine[(a * TT + c) * kPT] = acc[a][c];
+                for (int c = 0; c < TT; c++)
+                    mine[(a * TT + c) * kPT] = acc[a][c];
             if (!xmap) __threadfence();  // a reader on any XCD: write the partial back past the L2
             __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
             if (tid == 0) {
                 const uint64_t prev = __hip_atomic_fetch_add(cnt + t, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                const bool last = prev == others || (xmap && xcd_arrived(prev) == (uint32_t)(n_contrib - 1));
-                if (last) __hip_atomic_store(cnt + t, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                lflag = last ? 1 + (prev != others) : 0;
+                lflag = xcd_last(prev, one, (uint32_t)n_contrib);
+                if (lflag) __hip_atomic_store(cnt + t, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             __syncthreads();
             fl = __builtin_amdgcn_readfirstlane(lflag);

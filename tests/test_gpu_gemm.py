@@ -495,13 +495,17 @@ def test_gemm_prefill_int8_slices(miq, oracle, dev, qt, TB, N, K, switch):
 
 
 @pytest.mark.parametrize("qt,TB,N,K", [(Q8_0, 130, 1100, 5376), (Q8_0, 333, 5120, 4096), (Q4_K, 130, 2100, 2304), (Q5_K, 77, 4400, 5120),
-                                       (Q6_K, 256, 3000, 1024)])
-def test_prefill_partials_across_xcds(miq, oracle, dev, qt, TB, N, K, switch):
-    """Both prefill GEMMs where every second workgroup that shares a tile takes itself
-    for one on another XCD (XCD_ASTRAY): the last of the tile computes it again.  Within
-    the per-output bound in every run, with the normal placement's bits back afterwards."""
+                                       (Q6_K, 256, 3000, 1024), (Q4_K, 16, 5120, 17408), (Q4_K, 20, 300, 1024), (Q5_K, 9, 700, 2304),
+                                       (Q6_K, 16, 2050, 5120), (Q8_0, 33, 260, 2112), (Q8_0, 64, 1024, 5120)])
+def test_partials_across_xcds(miq, oracle, dev, qt, TB, N, K, switch):
+    """Both prefill GEMMs and the split-K 16-token kernel where every second workgroup that
+    shares a tile takes itself for one on another XCD (XCD_ASTRAY): the last of the tile
+    computes it again, in the 16-token kernel it reads the partials past its L2 (the
+    same bits).  Within the per-output bound in every run, with the normal placement's
+    bits back afterwards."""
     import torch
-    print(f"prefill across XCDs qt={qt} TB={TB} N={N} K={K}", flush=True)
+    print(f"partials across XCDs qt={qt} TB={TB} N={N} K={K}", flush=True)
+    again = TB > 64
     switch("PREFILL_FP16", "2")
     wq = weights(miq, qt, N, K, seed=TB + N)
     rng = np.random.default_rng(TB + K)
@@ -527,7 +531,7 @@ def test_prefill_partials_across_xcds(miq, oracle, dev, qt, TB, N, K, switch):
         got = run()
         assert_elem(got, exp, bound, residual=res)
         differ += int((got != normal).sum())
-    assert differ  # some tile was computed in one sum
+    assert bool(differ) == again  # a prefill tile is computed in one sum
     switch("XCD_ASTRAY", "0")
     assert np.array_equal(run().view(np.uint32), normal.view(np.uint32))
 
