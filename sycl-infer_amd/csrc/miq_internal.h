@@ -57,10 +57,10 @@ int launch_mfma16(hipStream_t stream, const miq_seg *s, int TB);
 int launch_mfma16_multi(hipStream_t stream, const miq_seg *segs, int n_segs, int TB);
 int launch_mfma16_dots(hipStream_t stream, const miq_seg *s, int TB, int32_t *out);
 
-// LDS-tiled int8-MFMA GEMM for prefill-sized batches (Q4_K, Q5_K, Q8_0)
+// LDS-tiled int8-MFMA GEMM for prefill-sized batches, with K slices where the tiles
+// leave CUs idle (Q8_0; the other types with PREFILL_FP16=0)
 bool mfma32_serves(const miq_seg *s);
-// Q6_K: the tiled kernel has no K split, so it takes a batch only when its
-// tiles cover every CU (else the split-K 16-token kernel is faster)
+// Q6_K: whether its tiles cover every CU (else the split-K 16-token kernel takes the batch)
 bool mfma32_fills(const miq_seg *s, int TB);
 // Q8_0: whether it beats the 16-token kernel at this shape
 bool mfma32_prefers(const miq_seg *s, int TB);

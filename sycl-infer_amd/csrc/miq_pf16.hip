@@ -21,9 +21,12 @@
 // 32 rows and all tokens, and decodes its own weights straight into operand
 // registers (two permlane swaps spread a row's 16-byte pieces over the four
 // lanes of the operand), so no weight passes through LDS and a decoded weight
-// serves 16*TT tokens.  The records stream into an LDS ring by direct loads two
-// 128-value stages ahead, one barrier per stage; weights come one block ahead
-// in registers.
+// serves 16*TT tokens.  The records stream into an LDS ring by direct loads issued
+// two 128-value stages ahead, one barrier per stage; weights are loaded one block
+// ahead into registers.  At a block's end the compiler waits for the weights
+// (vmcnt(0), for the copies of the loop-carried ones; every Q4_K and Q5_K form, Q6_K
+// from TT = 8 on), and so for the stages in flight too: the ring is worth about one
+// stage there.
 //
 // What bounds it: the instruction issue of the two waves per SIMD -- per
 // 32-value group a wave issues 8*TT fp32 fmas and 2*TT MFMAs, and the two
@@ -37,7 +40,7 @@
 // 512 / 1024 tokens 56 / 83 / 143 / 269 us; the form that decoded through LDS
 // with two barriers per 64 values took 91 / 125 / 190 us at 128 / 256 / 512.
 // Q6_K 5120 x 17408 (two planes, two MFMAs per group): 512 tokens 210 us, before
-// 273; 128 tokens 100 us, before 149.
+// 273; 128 tokens 100 us, before 149; at TT = 6, 7 and 8 it spills 2 to 13 registers.
 #include <type_traits>
 #include <utility>
 
@@ -960,9 +963,10 @@ static int pf_tile(int TB, int *mt) {
 //   this kernel      a + (t0 + t1 * TT) * B + TT / 4 * C
 // B = 256-value blocks of 256 x 16*TT tiles per workgroup, C = workgroups that
 // share a tile (2 where the tiles outnumber them), each but the last leaving a
-// partial that the last adds.  At 17408 x 5120 Q4_K the lines cross between 32
-// tokens (31 against 29 us) and 48 (37 against 51), at 7168 x 5120 Q5_K between
-// 96 (40 / 35) and 128, at 3584 x 1024 past 512 (31 / 23).
+// partial that the last adds.  At 17408 x 5120 Q4_K the lines cross at 32 tokens
+// (29.8 against 30.4 us; 33 tokens 33.5 / 52.7), at 7168 x 5120 Q5_K between 128
+// (one tile that nine workgroups share, 47.2 / 45.5) and 129 (two, 38.5 / 49.7), at
+// 3584 x 1024 past 512 (30.1 / 26.3).
 bool pf16_prefers(const miq_seg *s, int TB) {
     int n_cu = 0, mt = 0;
     if (device_cus(&n_cu) != MIQ_OK) n_cu = 256;
